@@ -96,7 +96,6 @@ __global__ void __launch_bounds__(256)
     constexpr int D = RHS::D, F = 3 + D;
     r8_init();
     const bg_ensemble_desc &d = ad->base;
-    const int lane = __lane_id();
     const uint64_t n = d.n;
     const uint32_t K = ad->checkpoint_every ? ad->checkpoint_every : 16u;
     const uint32_t maxck = ad->max_checkpoints ? ad->max_checkpoints : 128u;
@@ -105,85 +104,88 @@ __global__ void __launch_bounds__(256)
     const double *obs = stage_obs<OBS_LDS>(obs_lds, ad->obs_t, n_obs);
     RkLane<RHS, Tab> L;
     int64_t inst = -1;
-    uint32_t attempts = 0, nacc = 0, nrej = 0, next_stop = 0, n_stops = 0, nck = 0;
+    uint64_t k = first_position();
+    bool take = true, drained = ws.counters == nullptr;
+    uint32_t budget = kAdjMaxAttempts;
+    uint32_t attempts = 0, nacc = 0, next_stop = 0, n_stops = 0, nck = 0;
     uint32_t ck_left = K;  // accepted steps until the next checkpoint
     double target = 0.0;  // the next stop, else the end
     for (;;) {
-        const uint64_t need = __ballot(inst == -1);
-        if (need != 0) {
-            const int leader = __ffsll((unsigned long long)need) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&ws.counters[0], (uint32_t)__popcll(need));
-            base = __shfl(base, leader);
-            if (inst == -1) {
-                const uint64_t k = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane) - 1ull));
-                if (k < n) {
-                    inst = d.order ? (int64_t)gptr(d.order)[k] : (int64_t)k;
-                    const uint64_t i = (uint64_t)inst;
+        int st = -1;
+        if (take) {
+            inst = -1;
+            if (k < n) {
+                inst = d.order ? (int64_t)gptr(d.order)[k] : (int64_t)k;
+                const uint64_t i = (uint64_t)inst;
 #pragma unroll
-                    for (int c = 0; c < D; ++c) L.y[c] = gptr(d.y0)[c * n + i];
+                for (int c = 0; c < D; ++c) L.y[c] = gptr(d.y0)[c * n + i];
 #pragma unroll
-                    for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
-                    L.t = d.t0 ? gptr(d.t0)[i] : d.t0_s;
-                    L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
-                    L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
-                    L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
-                    L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
-                    L.dt = (L.dt_max + L.dt_min) * 0.5;
-                    attempts = nacc = nrej = next_stop = 0;
-                    ck_left = K;
-                    n_stops = count_stops(obs, n_obs, L.end);
-                    target = n_stops > 0 ? obs[0] : L.end;
-                    // checkpoint 0: the initial state
-                    double *ck0 = ws.ck + i * maxck * F;
-                    ck0[0] = L.t;
-                    ck0[1] = L.dt;
-                    ck0[2] = 0.0;
+                for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
+                L.t = d.t0 ? gptr(d.t0)[i] : d.t0_s;
+                L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
+                L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
+                L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
+                L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
+                L.dt = (L.dt_max + L.dt_min) * 0.5;
+                attempts = nacc = next_stop = 0;
+                ck_left = K;
+                n_stops = count_stops(obs, n_obs, L.end);
+                target = n_stops > 0 ? obs[0] : L.end;
+                // checkpoint 0: the initial state
+                double *ck0 = ws.ck + i * maxck * F;
+                ck0[0] = L.t;
+                ck0[1] = L.dt;
+                ck0[2] = 0.0;
 #pragma unroll
-                    for (int c = 0; c < D; ++c) ck0[3 + c] = L.y[c];
-                    nck = 1;
-                } else {
-                    inst = -2;
-                }
+                for (int c = 0; c < D; ++c) ck0[3 + c] = L.y[c];
+                nck = 1;
+                if (L.t >= L.end) st = BG_OK;
+                L.set_range(target);
+                L.head(target);
             }
         }
-        if (__ballot(inst >= 0) == 0) break;
-        int st = -1;
+        const int active = __popcll(ballot(inst >= 0));
+        if (active == 0) break;
+        const int want = drained ? active : 1;
         for (;;) {
-            if (__ballot(inst >= 0 && st >= 0) != 0) break;
+            const uint64_t running = ballot(inst >= 0 && st < 0);
+            if (active - __popcll(running) >= want) break;
+            uint32_t made = 0;
             if (inst >= 0 && st < 0) {
-                if (L.t >= L.end) {
-                    st = BG_OK;
-                } else if (attempts >= kAdjMaxAttempts) {
-                    st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
-                } else {
+                bool failed;
+                uint64_t at_end, fail, full, out;
+                do {
                     const bool to_stop = next_stop < n_stops;
-                    bool clamped;
-                    double h;
-                    const int r = L.attempt_to(target, to_stop, clamped, h);
-                    ++attempts;
-                    if (r == STEP_ACCEPTED) {
+                    const double dt_proposed = L.dt, h = L.h;
+                    uint32_t step = 0;
+                    const bool accepted = L.attempt(failed, step);
+                    const bool at_stop = accepted && L.clamped && to_stop;
+                    // a step cut short by a stop hands on the size proposed
+                    // before the cut (as in the path kernel)
+                    if (at_stop) L.dt = fmax(L.dt, dt_proposed);
+                    const bool low = L.dt < L.dt_min && L.t < L.end;
+                    bool no_room = false;
+                    if (accepted && !low) {
                         const uint64_t i = (uint64_t)inst;
                         // accepted step nacc lies in segment nacc / K < maxck
                         // (the capacity test below ends the solve at the
                         // segment boundary past the last checkpoint)
-                        ws.hs[i * maxck * K + nacc] = (clamped && to_stop) ? -h : h;
+                        ws.hs[i * maxck * K + nacc] = at_stop ? -h : h;
                         ++nacc;
-                        if (clamped && to_stop) {
+                        if (at_stop) {
                             L.t = target;
 #pragma unroll
                             for (int c = 0; c < D; ++c)
                                 ws.res[(i * n_obs + next_stop) * D + c] = L.y[c];
                             ++next_stop;
                             target = next_stop < n_stops ? obs[next_stop] : L.end;
+                            L.set_range(target);
                         }
                         --ck_left;
-                        if (L.t >= L.end) {
-                            st = BG_OK;
-                        } else if (ck_left == 0) {
+                        if (ck_left == 0 && !(L.t >= L.end)) {
                             ck_left = K;
                             if (nck >= maxck) {
-                                st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
+                                no_room = true;
                             } else {
                                 double *ckp = ws.ck + (i * maxck + nck) * F;
                                 ckp[0] = L.t;
@@ -194,15 +196,31 @@ __global__ void __launch_bounds__(256)
                                 ++nck;
                             }
                         }
-                    } else if (r == STEP_REJECTED) {
-                        ++nrej;
-                    } else {
-                        st = r;
                     }
-                }
+                    L.head(target);
+                    ++made;
+                    at_end = ballot(L.t >= L.end);
+                    fail = ballot(low);
+                    full = ballot(no_room);
+                    out = at_end | fail | full;
+                    if constexpr (kRhsFails<RHS>) out |= ballot(failed);
+                } while (out == 0 && made < budget);
+                attempts += made;
+                if (failed)
+                    st = BG_USER_ERROR;
+                else if (lane_bit(fail))
+                    st = BG_MINIMUM_TIME_DELTA_EXCEEDED;
+                else if (lane_bit(at_end))
+                    st = BG_OK;
+                else if (lane_bit(full) || attempts >= kAdjMaxAttempts)
+                    st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
             }
+            budget -= first_of(made, running);
+            if (budget == 0)
+                budget = kAdjMaxAttempts - wave_max_u32(inst >= 0 && st < 0 ? attempts : 0u);
         }
-        if (inst >= 0 && st >= 0) {
+        take = inst >= 0 && st >= 0;
+        if (take) {
             const uint64_t i = (uint64_t)inst;
             // an observation at the end time (after the last stop) scores the
             // final state
@@ -223,11 +241,17 @@ __global__ void __launch_bounds__(256)
             if (d.counts) {
                 bg_counts cc;
                 cc.n_accepted = nacc;
-                cc.n_rejected = nrej;
+                // an attempt that ended in a failure counts as neither
+                cc.n_rejected =
+                    attempts - nacc -
+                    (st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u);
                 d.counts[i] = cc;
             }
             inst = -1;
         }
+        if (drained) break;
+        const uint64_t need = ballot(take);
+        k = next_position(ws.counters, need, n, drained);
     }
 }
 
@@ -363,7 +387,6 @@ __global__ void __launch_bounds__(256)
     extern __shared__ double tape_lds[];
     r8_init();
     const bg_ensemble_desc &d = ad->base;
-    const int lane = __lane_id();
     const uint64_t slot = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t n = d.n;
     double *const tape = LDS_TAPE ? tape_lds + threadIdx.x : ws.seg + slot;
@@ -411,47 +434,42 @@ __global__ void __launch_bounds__(256)
             for (int c = 0; c < D; ++c) rn[c] = ws.res[(i * n_obs + (uint64_t)k) * D + c];
         }
     };
+    uint64_t k = first_position();
+    bool take = true, drained = ws.counters == nullptr;
     for (;;) {
-        const uint64_t need = __ballot(inst == -1);
-        if (need != 0) {
-            const int leader = __ffsll((unsigned long long)need) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&ws.counters[1], (uint32_t)__popcll(need));
-            base = __shfl(base, leader);
-            if (inst == -1) {
-                const uint64_t k = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane) - 1ull));
-                if (k < n) {
-                    inst = (int64_t)ws.order_b[k];
-                    const uint64_t i = (uint64_t)inst;
+        if (take) {
+            inst = -1;
+            if (k < n) {
+                inst = (int64_t)ws.order_b[k];
+                const uint64_t i = (uint64_t)inst;
 #pragma unroll
-                    for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
-                    L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
-                    L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
-                    L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
-                    L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
+                for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
+                L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
+                L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
+                L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
+                L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
 #pragma unroll
-                    for (int c = 0; c < P; ++c) pb[c] = 0.0;
-                    n_stops = count_stops(obs, n_obs, L.end);
-                    const bool final_obs = n_stops < n_obs && obs[n_stops] == L.end;
+                for (int c = 0; c < P; ++c) pb[c] = 0.0;
+                n_stops = count_stops(obs, n_obs, L.end);
+                const bool final_obs = n_stops < n_obs && obs[n_stops] == L.end;
 #pragma unroll
-                    for (int c = 0; c < D; ++c)
-                        lam[c] = final_obs ? 2.0 * ws.res[(i * n_obs + n_stops) * D + c] : 0.0;
-                    const int fw = d.status ? gptr(d.status)[i] : BG_OK;
-                    seg = fw == BG_OK ? (int)ws.nck[i] - 1 : -1;
-                    load_res((int)n_stops - 1, i);
-                    if (seg >= 0) {
-                        load_ck(seg, i);
-                        load_h(seg, i);
-                    }
-                } else {
-                    inst = -2;
+                for (int c = 0; c < D; ++c)
+                    lam[c] = final_obs ? 2.0 * ws.res[(i * n_obs + n_stops) * D + c] : 0.0;
+                const int fw = d.status ? gptr(d.status)[i] : BG_OK;
+                seg = fw == BG_OK ? (int)ws.nck[i] - 1 : -1;
+                load_res((int)n_stops - 1, i);
+                if (seg >= 0) {
+                    load_ck(seg, i);
+                    load_h(seg, i);
                 }
             }
         }
-        if (__ballot(inst >= 0) == 0) break;
+        const int active = __popcll(ballot(inst >= 0));
+        if (active == 0) break;
+        const int want = drained ? active : 1;
         bool fin = false;
         for (;;) {
-            if (__ballot(inst >= 0 && fin) != 0) break;
+            if (__popcll(ballot(inst >= 0 && fin)) >= want) break;
             if (inst >= 0 && !fin) {
                 if (seg < 0) {
                     fin = true;
@@ -530,7 +548,8 @@ __global__ void __launch_bounds__(256)
                 }
             }
         }
-        if (inst >= 0 && fin) {
+        take = inst >= 0 && fin;
+        if (take) {
             const uint64_t i = (uint64_t)inst;
             const int fw = d.status ? gptr(d.status)[i] : BG_OK;
             const double nan = __builtin_nan("");
@@ -545,13 +564,17 @@ __global__ void __launch_bounds__(256)
             }
             inst = -1;
         }
+        if (drained) break;
+        const uint64_t need = ballot(take);
+        k = next_position(ws.counters + 1, need, n, drained);
     }
 }
 
-__global__ void adj_setup_kernel(uint32_t *counters, bg_adjoint_desc *dst, const bg_adjoint_desc d) {
+__global__ void adj_setup_kernel(uint32_t *counters, uint32_t lanes_f, uint32_t lanes_b,
+                                 bg_adjoint_desc *dst, const bg_adjoint_desc d) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        counters[0] = 0u;
-        counters[1] = 0u;
+        counters[0] = lanes_f;
+        counters[1] = lanes_b;
         *dst = d;
     }
 }
@@ -653,7 +676,8 @@ int rk_launch_adjoint(int method, int rhs, const bg_adjoint_desc &ad, hipStream_
         q = align(q + sizeof(uint32_t) * n);
         void *sort_tmp = q;
         ws.order_b = order_b;
-        adj_setup_kernel<<<1, 64, 0, stream>>>(ws.counters, dd, ad);
+        adj_setup_kernel<<<1, 64, 0, stream>>>(ws.counters, (uint32_t)(grid_f * 256),
+                                              (uint32_t)(grid_b * 256), dd, ad);
         fwd<<<(uint32_t)grid_f, 256, 0, stream>>>(dd, ws);
         // residuals through LDS tiles when a tile fits 64 KiB (n_obs <= 25
         // at D = 2 … kResTile x n_obs x D doubles)

@@ -274,10 +274,18 @@ __host__ __device__ constexpr double root8_scale(int b) {
 
 // The eight scales in LDS for kernels that call root8_lds(): a per-lane
 // table read replaces three select pairs and two products.  r8_init() fills
-// it at kernel entry (every thread of the block must call it).
+// it at kernel entry (every thread of the block must call it).  Entry k is
+// the scale of the arguments whose biased exponent is k mod 8, times 2^-128
+// (a power of two, so every product with it rounds like one with the scale):
+// root8_lds() then takes the entry and the final exponent straight from the
+// argument's high word.
 __shared__ double r8_table[8];
 __device__ __forceinline__ void r8_init() {
-    if (threadIdx.x < 8) r8_table[threadIdx.x] = root8_scale((int)threadIdx.x);
+    // r = m 2^e, m in [1, 2), has the biased exponent e + 1023
+    if (threadIdx.x < 8) {
+        const int b = (int)((threadIdx.x + 1) & 7);  // e mod 8
+        r8_table[threadIdx.x] = root8_scale(b) * (b == 0 ? 0x1p-127 : 0x1p-128);
+    }
     __syncthreads();
 }
 
@@ -286,22 +294,10 @@ constexpr double kRoot8Poly[6] = {0.0029682975037312034, -0.005693672682686368,
                                   0.010621966427993313,  -0.025512534910039072,
                                   0.08766623673998887,   1.0519887150881322};
 
-// c: kRoot8Poly, each through an SGPR pair (kc) for the three-address fma.
-__device__ __forceinline__ double root8_poly(double r, int &e, const double (&c)[6]) {
-    int ex;
-    const double mant = frexp(r, &ex);
-    // mant * 2 is exact, so the fused form rounds like mul-then-add
-    const double x = fma(mant, 2.0, -1.5);
-    e = ex - 1;
-    double p = c[0];
-#pragma unroll
-    for (int k = 1; k < 6; ++k) p = fma(p, x, c[k]);
-    return p;
-}
-
 __device__ __forceinline__ double root8_poly(double r, int &e) {
     int ex;
     const double mant = frexp(r, &ex);
+    // mant * 2 is exact, so the fused form rounds like mul-then-add
     const double x = fma(mant, 2.0, -1.5);
     e = ex - 1;
     // coefficients through SGPRs: three-address fma, no accumulator copies
@@ -317,17 +313,20 @@ __device__ __forceinline__ double root8(double r) {
     return ldexp(p * root8_scale(e & 7), e >> 3);
 }
 
-// The same value with the scale read from r8_table.
+// The same value for r in (1e-8, 65536), the scale read from r8_table: the
+// entry by the three low bits of the biased exponent, the final exponent its
+// other bits (the -128 in the table brings (e + 1023) >> 3 back to e >> 3,
+// the entry that belongs to e mod 8 = 0 one more, because 1023 = 8 * 127 + 7).
+// c: kRoot8Poly.  Anything outside that range gives an unused value.
 __device__ __forceinline__ double root8_lds(double r, const double (&c)[6]) {
-    int e;
-    const double p = root8_poly(r, e, c);
-    return ldexp(p * r8_table[e & 7], e >> 3);
-}
-
-__device__ __forceinline__ double root8_lds(double r) {
-    int e;
-    const double p = root8_poly(r, e);
-    return ldexp(p * r8_table[e & 7], e >> 3);
+    const uint32_t hi = (uint32_t)(__builtin_bit_cast(uint64_t, r) >> 32);
+    const double scale =
+        *(const double *)((const char *)r8_table + ((hi >> 17) & 0x38u));
+    const double x = fma(__builtin_amdgcn_frexp_mant(r), 2.0, -1.5);
+    double p = c[0];
+#pragma unroll
+    for (int k = 1; k < 6; ++k) p = fma(p, x, c[k]);
+    return ldexp(p * scale, (int)(hi >> 23));
 }
 
 // ---------------------------------------------------------------------------
@@ -353,15 +352,61 @@ __device__ __forceinline__ double qmin_s(double a, double b) {
     return r;
 }
 
+// The lanes (of those active) for which c holds.
+__device__ __forceinline__ uint64_t ballot(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+
+__device__ __forceinline__ bool lane_bit(uint64_t mask) { return (mask >> __lane_id()) & 1; }
+
+// v of the first lane of a non-empty mask, wave-uniform.
+__device__ __forceinline__ uint32_t first_of(uint32_t v, uint64_t mask) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, __ffsll((unsigned long long)mask) - 1);
+}
+
 // ---------------------------------------------------------------------------
-// One lane's RK state and one call of RungeKuttaSolver::step.
+// a / b correctly rounded, where the quotient lies in (1e-8, 65536) and a in
+// [2^-800, 2^800]: the hardware reciprocal (relative error below 2^-22),
+// one cubic refinement (error e^3), the product, its exact residual and one
+// correction (Markstein 1990).  Eight operations against the IEEE division's
+// eleven, which also scale for exponents that do not occur here.
 // ---------------------------------------------------------------------------
-enum : int { STEP_ACCEPTED = -1, STEP_REJECTED = -2 };
+__device__ __forceinline__ double div_mid(double a, double b) {
+    const double y0 = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, y0, 1.0);
+    const double y = fma(y0, fma(e, e, e), y0);
+    const double q = a * y;
+    return fma(fma(-b, q, a), y, q);
+}
+
+// Right-hand sides that can report a UserError.
+template <class RHS>
+inline constexpr bool kRhsFails = false;
+template <int D>
+inline constexpr bool kRhsFails<RhsFailAfter<D>> = true;
+
+// ---------------------------------------------------------------------------
+// One lane's RK state and one call of RungeKuttaSolver::step (rk.rs:361-423),
+// in two parts:
+//   head(target)  the step size h with the end clamp of rk.rs:366-368 aimed
+//                 at `target` and the first stage's right-hand side;
+//   attempt()     the stages, the error test, the controller and, if the
+//                 step is accepted, the update.
+// A loop calls head() for the next attempt right after attempt(): its dozen
+// independent operations then cover the latency of the loop's exit test.
+//
+// What bounds an attempt is the number of instructions it issues: a wave alone
+// on its SIMD issues one FP64 operation per ~5 cycles whether or not it
+// depends on the one before (measured: 5.2 cycles dependent, 5.1 in four
+// chains), two or more waves one per 4, and a branch around a few lanes' work
+// costs 30-40 (compare, exec update, jump).  So the ordinary attempt runs
+// straight through: the quotient without range scaling (div_mid), the root for
+// every lane, and one wave-uniform test that sends the lanes outside its range
+// to code off that line.
+// ---------------------------------------------------------------------------
 
 // HOIST: the tableau and root coefficients are put through SGPR pairs once,
 // where the lane state is declared, rather than at each use (see cm below);
-// for the persistent ensemble loop and the adjoint's backward replay, whose
-// SGPR budgets have room for them (in the adjoint's forward pass they would
+// for the persistent loops and the adjoint's backward replay, whose SGPR
+// budgets have room for them (in the adjoint's forward pass they would
 // double its SGPR spills).
 template <class RHS, class Tab, bool HOIST = false>
 struct RkLane {
@@ -370,6 +415,10 @@ struct RkLane {
     double y[D];
     double K[S][D];  // half_steps; persists across attempts (read by AS_BUILT)
     double p[RHS::P > 0 ? RHS::P : 1];
+    double h;        // the attempt's step size (head)
+    double F0[D];    // f(t, y) (head; not for right-hand sides that can fail)
+    double r_lo;     // 1e-8, or +inf: every quotient through the IEEE division
+    bool clamped;    // h was cut to reach the target
     // With HOIST, the stage coefficients, the first error weight and the
     // root's polynomial through SGPR pairs (kc), taken once where the lane
     // state is declared, so every attempt reads the pairs directly instead
@@ -391,6 +440,9 @@ struct RkLane {
             c_below_one = 0x1.fffffffffffffp-1;
 #pragma unroll
             for (int k = 0; k < 6; ++k) cr[k] = kc(kRoot8Poly[k]);
+            // one operand of the polynomial's first fma in a VGPR pair: an
+            // instruction reads at most one SGPR pair
+            asm("" : "+v"(cr[0]));
         }
     }
     __device__ __forceinline__ double coef_m(int i, int j) const {
@@ -398,53 +450,61 @@ struct RkLane {
         return kc(Tab::m(i, j));
     }
 
-    // rk.rs:361-423 without the Done test (the caller does it).  Returns
-    // STEP_ACCEPTED, STEP_REJECTED or an IVPError code.
-    __device__ __forceinline__ int attempt() {
-        bool clamped;
-        return attempt_to(end, false, clamped);
+    // Called when an instance is loaded and when the target changes: whether
+    // every quotient of the controller can take div_mid.  q2 = (tol h)^2 then
+    // lies in [2^-800, 2^800]: h is between dt_min and dt_max, or target - t,
+    // a multiple of 2^-153 unless the target lies within 2^-100 of zero.
+    __device__ __forceinline__ void set_range(double target) {
+        const bool mid = tol >= 0x1p-200 && tol <= 0x1p200 && dt_min >= 0x1p-200 &&
+                         dt_max <= 0x1p200 && fabs(target) >= 0x1p-100;
+        r_lo = mid ? 1e-8 : __builtin_inf();
     }
 
-    // The same attempt with the end clamp of rk.rs:366-368 aimed at `target`
-    // (the end, or an observation time before it: `to_stop`); `clamped`
-    // reports whether dt was cut to reach it.  An accepted step cut short to
-    // land on a stop hands the next attempt at least the step size proposed
-    // before the cut: a stop just past an accepted time must not shrink dt
-    // below dt_min and fail a solve that succeeds without the stop (at the
-    // end the solve is done, so the reference clamp is unaffected).
-    __device__ __forceinline__ int attempt_to(double target, bool to_stop, bool &clamped) {
-        double h;
-        return attempt_to(target, to_stop, clamped, h);
+    __device__ __forceinline__ void head(double target) {
+        clamped = t + dt >= target;
+        h = clamped ? target - t : dt;
+        if constexpr (!kRhsFails<RHS>) (void)RHS::eval(fma(Tab::c(0), h, t), y, p, F0);
     }
 
     // The stages of a step of size h from (t, y): rk.rs:370-384.  False if
-    // the right-hand side reports an error.
-    __device__ __forceinline__ bool stages(double h) {
+    // the right-hand side reports an error.  HEAD: the first stage's
+    // right-hand side is in F0.
+    template <bool HEAD>
+    __device__ __forceinline__ bool stages(double hh) {
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             double Y[D];
 #pragma unroll
             for (int d = 0; d < D; ++d) Y[d] = y[d];
+            // the first row of a tableau read as built is not empty: its
+            // stage does not start from y
+            bool from_y = i == 0;
 #pragma unroll
             for (int j = 0; j < S; ++j) {
                 const double m = Tab::m(i, j);
                 if (m != 0.0) {
+                    from_y = false;
 #pragma unroll
                     for (int d = 0; d < D; ++d) Y[d] = fma(coef_m(i, j), K[j][d], Y[d]);
                 }
             }
-            const double ti = fma(Tab::c(i), h, t);
             double f[D];
-            if (!RHS::eval(ti, Y, p, f)) return false;
+            if (HEAD && !kRhsFails<RHS> && from_y) {
 #pragma unroll
-            for (int d = 0; d < D; ++d) K[i][d] = f[d] * h;
+                for (int d = 0; d < D; ++d) f[d] = F0[d];
+            } else {
+                const double ti = fma(Tab::c(i), hh, t);
+                if (!RHS::eval(ti, Y, p, f)) return false;
+            }
+#pragma unroll
+            for (int d = 0; d < D; ++d) K[i][d] = f[d] * hh;
         }
         return true;
     }
 
     // The accepted step's update from the stages: rk.rs:392-398.
-    __device__ __forceinline__ void update(double h) {
-        t += h;
+    __device__ __forceinline__ void update(double hh) {
+        t += hh;
 #pragma unroll
         for (int j = 0; j < S; ++j) {
             const double b = Tab::b(j);
@@ -455,28 +515,36 @@ struct RkLane {
         }
     }
 
-    // A step of size h known to be accepted (the replay of a recorded step):
-    // the operations of attempt_to's accepted branch, so (t, y) come out
+    // A step of size hh known to be accepted (the replay of a recorded step):
+    // the operations of an accepted attempt, so (t, y) come out
     // bit-identical, without the error estimate and the controller.  dt is
     // left as it was.
-    __device__ __forceinline__ bool advance(double h) {
-        if (!stages(h)) return false;
-        update(h);
+    __device__ __forceinline__ bool advance(double hh) {
+        if (!stages<false>(hh)) return false;
+        update(hh);
         return true;
     }
 
-    // attempt_to that also reports the step size it tried in h (dt after
-    // the clamp).
-    __device__ __forceinline__ int attempt_to(double target, bool to_stop, bool &clamped,
-                                              double &h) {
-        clamped = false;
-        const double dt_proposed = dt;
-        if (t + dt >= target) {
-            dt = target - t;
-            clamped = true;
+    // The controller's factor for a quotient outside (r_lo, 65536), where the
+    // clamps delta <= 0.1 / delta >= 4 apply (r <= 1e-8 / r >= 65536), the
+    // quotient needs the IEEE division (see set_range) or it is NaN.  At
+    // 65536 and above only the quotient's size matters.
+    __device__ __forceinline__ static double factor_outside(double q2, double ss, double r_lo,
+                                                            double &r) {
+        if (r >= 65536.0 && r_lo < 1.0) return 4.0;
+        r = q2 / ss;
+        return r <= 1e-8 ? 0.1 : (r >= 65536.0 ? 4.0 : root8(r));
+    }
+
+    // One attempt of size h (head).  Returns whether it was accepted, and
+    // counts it in nacc then; failed is set if the right-hand side reported an
+    // error (then nothing else has changed but K).
+    __device__ __forceinline__ bool attempt(bool &failed, uint32_t &nacc) {
+        failed = false;
+        if (!stages<true>(h)) {
+            failed = true;
+            return false;
         }
-        h = dt;
-        if (!stages(dt)) return BG_USER_ERROR;
         // rk.rs:386-390
         double E[D];
         constexpr int e0 = Tab::e_first();
@@ -497,15 +565,22 @@ struct RkLane {
         // with q = tol*dt; delta = (tol/err)^(1/4) = r^(1/8), r = q^2/ss,
         // and the clamps delta <= 0.1 / delta >= 4 become r <= 1e-8 /
         // r >= 65536 (safety factor 100/100 = 1.0, rk.rs:266-268).
-        const double q = tol * dt;
+        const double q = tol * h;
         const double q2 = q * q;
         const bool accepted = ss <= q2;
-        const double r = q2 / ss;
+        double r = div_mid(q2, ss);
         double f0;
         if constexpr (HOIST) {
-            f0 = r <= 1e-8 ? 0.1 : (r >= 65536.0 ? 4.0 : root8_lds(r, cr));
+            f0 = root8_lds(r, cr);
         } else {
-            f0 = r <= 1e-8 ? 0.1 : (r >= 65536.0 ? 4.0 : root8_lds(r));
+            double c[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) c[k] = kc(kRoot8Poly[k]);
+            f0 = root8_lds(r, c);
+        }
+        const bool outside = !(r > r_lo && r < 65536.0);
+        if (__builtin_expect(ballot(outside) != 0, 0)) {
+            if (outside) f0 = factor_outside(q2, ss, r_lo, r);
         }
         // near r = 1 the sign of delta - 1 ~ (r - 1)/8 is far below root8's
         // error: bound by the tangent 1 + (r - 1)/8 (r^(1/8) is concave, the
@@ -516,31 +591,40 @@ struct RkLane {
         // into the attempt cap (the reference retries forever).
         const double tang = fma(r - 1.0, 0.125, 1.0);
         const double f = qmin(f0, tang);
-        const double fa = qmax_one(f);
-        const double fr = HOIST ? qmin(f, c_below_one) : qmin_s(f, 0x1.fffffffffffffp-1);
-        const double factor = accepted ? fa : fr;
-        if (accepted) update(dt);
+        double factor = HOIST ? qmin(f, c_below_one) : qmin_s(f, 0x1.fffffffffffffp-1);
+        if (accepted) {
+            update(h);
+            ++nacc;
+            factor = qmax_one(f);
+        }
         // dt is never NaN here (factor is finite), so the clamp is a minimum
-        dt = qmin(dt * factor, dt_max);
-        if (accepted && clamped && to_stop) dt = fmax(dt, dt_proposed);
-        // rk.rs:414-416
-        if (dt < dt_min && t < end) return BG_MINIMUM_TIME_DELTA_EXCEEDED;
-        return accepted ? STEP_ACCEPTED : STEP_REJECTED;
+        dt = qmin(h * factor, dt_max);
+        return accepted;
     }
 };
 
-// The descriptor's device-memory copy, read at the point of use.  The empty
-// asm hides the pointer's value from the optimiser, so the loads are not
-// hoisted out of the persistent loop (no ~30 descriptor registers live across
-// the attempts) while staying ordinary cached loads that issue together under
-// one wait.  (Volatile reads would be uncached, each waited for in turn.)
-__device__ __forceinline__ const bg_ensemble_desc *desc_at_use(const bg_ensemble_desc *dv) {
+// The descriptor, read at the point of use.  The empty asm hides the
+// pointer's value from the optimiser, so the loads are not hoisted out of the
+// persistent loop (no ~30 descriptor registers live across the attempts)
+// while staying ordinary cached loads that issue together under one wait.
+// (Volatile reads would be uncached, each waited for in turn.)
+template <class DP>
+__device__ __forceinline__ DP desc_at_use(DP dv) {
     asm volatile("" : "+s"(dv));
     return dv;
 }
 
-__device__ __forceinline__ bg_ensemble_desc desc_inputs(const bg_ensemble_desc *dv_) {
-    const bg_ensemble_desc *dv = desc_at_use(dv_);
+// A kernel whose first parameter is the descriptor by value reads it from its
+// argument segment (constant memory, scalar loads): no copy in device memory
+// and no kernel before it to make one.
+typedef const __attribute__((address_space(4))) bg_ensemble_desc *karg_desc;
+__device__ __forceinline__ karg_desc kernarg_desc() {
+    return (karg_desc)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+template <class DP>
+__device__ __forceinline__ bg_ensemble_desc desc_inputs(DP dv_) {
+    const DP dv = desc_at_use(dv_);
     bg_ensemble_desc d;
     d.n = dv->n;
     d.order = dv->order;
@@ -559,8 +643,9 @@ __device__ __forceinline__ bg_ensemble_desc desc_inputs(const bg_ensemble_desc *
     return d;
 }
 
-__device__ __forceinline__ bg_ensemble_desc desc_outputs(const bg_ensemble_desc *dv_) {
-    const bg_ensemble_desc *dv = desc_at_use(dv_);
+template <class DP>
+__device__ __forceinline__ bg_ensemble_desc desc_outputs(DP dv_) {
+    const DP dv = desc_at_use(dv_);
     bg_ensemble_desc d;
     d.n = dv->n;
     d.t_out = dv->t_out;
@@ -569,6 +654,42 @@ __device__ __forceinline__ bg_ensemble_desc desc_outputs(const bg_ensemble_desc 
     d.counts = dv->counts;
     d.work = dv->work;
     return d;
+}
+
+// ---------------------------------------------------------------------------
+// The work queue of a persistent launch.  Lane g of the grid starts with
+// schedule position g; positions from the number of lanes on are handed out by
+// a counter that starts there (one atomicAdd per wave).  A launch whose
+// positions all have a lane passes no counter: nothing to set up before it,
+// and no wave asks for more.  Once a wave has been told that the positions are
+// used up it runs its remaining lanes to their ends without asking again, and
+// stores them together.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint64_t first_position() {
+    return (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+}
+// positions for the lanes of `need`; drained (wave-uniform) is set once the
+// counter has passed n
+__device__ __forceinline__ uint64_t next_position(uint32_t *counter, uint64_t need, uint64_t n,
+                                                  bool &drained) {
+    const int lane = __lane_id();
+    const int leader = __ffsll((unsigned long long)need) - 1;
+    const uint32_t cnt = (uint32_t)__popcll(need);
+    uint32_t base = 0;
+    if (lane == leader) base = atomicAdd(counter, cnt);
+    base = first_of(base, need);
+    drained = (uint64_t)base + cnt >= n;
+    return (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane) - 1ull));
+}
+
+// The largest value over the wave's lanes, wave-uniform (every lane active).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)v, m);
+        v = o > v ? o : v;
+    }
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
 }  // namespace bg

@@ -11,8 +11,9 @@
 //  * inputs and outputs are structure-of-arrays in HBM ([component][n]);
 //  * the launch is persistent (grid = resident blocks); a wave refills its
 //    idle lanes from a global work counter with one atomicAdd per wave
-//    (ballot + popcount + mbcnt rank), so finished instances retire without
-//    stalling the other lanes;
+//    (ballot + popcount rank), so finished instances retire without
+//    stalling the other lanes; an ensemble that fits the resident lanes needs
+//    no counter (first_position, next_position in bg_device.h);
 //  * an optional schedule permutation hands out instances longest-first.
 #include "bg_device.h"
 #include "bg_internal.h"
@@ -20,13 +21,17 @@
 namespace bg {
 
 static constexpr uint64_t kDefaultMaxAttempts = 10000000ull;
-static constexpr int64_t kNeedWork = -1;
-static constexpr int64_t kExhausted = -2;
+static constexpr int64_t kNoInstance = -1;
 
 template <class T>
 struct Tag {
     using type = T;
 };
+
+__device__ __forceinline__ uint32_t attempt_cap(uint64_t max_attempts) {
+    return (uint32_t)((max_attempts && max_attempts < kDefaultMaxAttempts) ? max_attempts
+                                                                           : kDefaultMaxAttempts);
+}
 
 template <class RHS, class Tab, bool H>
 __device__ __forceinline__ void rk_load(RkLane<RHS, Tab, H> &L, const bg_ensemble_desc &d,
@@ -47,6 +52,7 @@ __device__ __forceinline__ void rk_load(RkLane<RHS, Tab, H> &L, const bg_ensembl
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int k = 0; k < D; ++k) L.K[s][k] = 0.0;  // rk.rs:323-327
+    L.set_range(L.end);
 }
 
 template <class RHS, class Tab, bool H>
@@ -69,84 +75,121 @@ __device__ __forceinline__ void rk_store(const RkLane<RHS, Tab, H> &L, const bg_
 }
 
 // One attempt plus the iterator's bookkeeping.  Returns -1 to continue, or
-// the final status (BG_OK at Done).
+// the final status (BG_OK at Done).  For the single-lane kernels.
 template <class RHS, class Tab, bool H>
 __device__ __forceinline__ int rk_advance(RkLane<RHS, Tab, H> &L, uint32_t &attempts, uint32_t cap,
                                           uint32_t &nacc, uint32_t &nrej) {
     if (attempts >= cap) return BG_MAXIMUM_ITERATIONS_EXCEEDED;
-    const int st = L.attempt();
+    bool failed;
+    L.head(L.end);
+    uint32_t step = 0;
+    const bool accepted = L.attempt(failed, step);
     ++attempts;
-    if (st == STEP_ACCEPTED) {
+    if (failed) return BG_USER_ERROR;
+    // rk.rs:414-416
+    if (L.dt < L.dt_min && L.t < L.end) return BG_MINIMUM_TIME_DELTA_EXCEEDED;
+    if (accepted) {
         ++nacc;
         // the iterator's next step() call would return Done (rk.rs:362-364)
         return L.t >= L.end ? BG_OK : -1;
     }
-    if (st == STEP_REJECTED) {
-        ++nrej;
-        return -1;
-    }
-    return st;
+    ++nrej;
+    return -1;
 }
 
 // Persistent ensemble kernel.  Outer loop: refill idle lanes (one atomicAdd
 // per wave), store finished instances.  Inner loop: step attempts until at
-// least `refill_min` lanes of the wave have finished (or all have).  Waves
-// holding an instance among the first `prio_cutoff` schedule positions run at
-// raised wave priority so the longest solves are not starved.
+// least `refill_min` lanes of the wave have finished, or, once the queue is
+// used up, all have.  Waves holding an instance among the first `prio_cutoff`
+// schedule positions run at raised wave priority so the longest solves are
+// not starved.
+//
+// The attempt loop holds no more bookkeeping than the accepted count and one
+// wave-uniform exit test (a lane at its end or below dt_min, or the attempt
+// budget that the wave's lanes share until the first could reach its cap);
+// statuses and attempt counts are settled outside it.  Lorenz-63 RK45: 193 ->
+// 171 vector instructions per attempt.
 template <class RHS, class Tab>
 __global__ void __launch_bounds__(256)
-    rk_ensemble_kernel(const bg_ensemble_desc *dv, uint32_t *__restrict__ counter,
+    rk_ensemble_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter,
                        uint32_t refill_min, uint32_t prio_cutoff) {
     r8_init();
+    const karg_desc dv = kernarg_desc();
     RkLane<RHS, Tab, true> L;
-    const int lane = __lane_id();
-    const uint64_t max_att = dv->max_attempts;
-    const uint32_t cap = (uint32_t)((max_att && max_att < kDefaultMaxAttempts) ? max_att
-                                                                                : kDefaultMaxAttempts);
-    int64_t inst = kNeedWork;
-    uint64_t pos = 0;
-    uint32_t attempts = 0, nacc = 0, nrej = 0;
+    const uint32_t cap = attempt_cap(dv->max_attempts);
+    uint32_t budget = cap;  // attempts until a lane could reach the cap
+    bool drained = counter == nullptr;
+    int64_t inst = kNoInstance;
+    uint64_t pos = first_position();
+    bool take = true;
+    uint32_t attempts = 0, nacc = 0;
     for (;;) {
         // ---- refill --------------------------------------------------------
-        const uint64_t need = __ballot(inst == kNeedWork);
-        if (need != 0) {
-            const int leader = __ffsll((unsigned long long)need) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(need));
-            base = __shfl(base, leader);
-            if (inst == kNeedWork) {
-                const uint64_t below = need & ((1ull << lane) - 1ull);
-                pos = (uint64_t)base + (uint64_t)__popcll(below);
-                const bg_ensemble_desc di = desc_inputs(dv);  // one batch of loads
-                if (pos < di.n) {
-                    inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
-                    rk_load(L, di, (uint64_t)inst);
-                    attempts = nacc = nrej = 0;
-                } else {
-                    inst = kExhausted;
+        int st = -1;  // running; >= 0: the instance's status
+        if (take) {
+            const bg_ensemble_desc di = desc_inputs(dv);  // one batch of loads
+            inst = kNoInstance;
+            if (pos < di.n) {
+                inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
+                rk_load(L, di, (uint64_t)inst);
+                attempts = nacc = 0;
+                if (L.t >= L.end) st = BG_OK;  // Done before any step
+                L.head(L.end);
+            }
+        }
+        if (prio_cutoff) {
+            if (__ballot(inst >= 0 && pos < prio_cutoff) != 0)
+                __builtin_amdgcn_s_setprio(2);
+            else
+                __builtin_amdgcn_s_setprio(0);
+        }
+        const int active = __popcll(ballot(inst >= 0));
+        if (active == 0) break;
+        // ---- attempts ------------------------------------------------------
+        const int want = drained ? active : min((int)refill_min, active);
+        for (;;) {
+            const uint64_t running = ballot(inst >= 0 && st < 0);
+            if (active - __popcll(running) >= want) break;
+            uint32_t made = 0;
+            if (inst >= 0 && st < 0) {
+                bool accepted, failed;
+                uint64_t at_end, low, out;
+                do {
+                    accepted = L.attempt(failed, nacc);
+                    L.head(L.end);
+                    ++made;
+                    at_end = ballot(L.t >= L.end);
+                    low = ballot(L.dt < L.dt_min);
+                    out = at_end | low;
+                    if constexpr (kRhsFails<RHS>) out |= ballot(failed);
+                } while (out == 0 && made < budget);
+                attempts += made;
+                if (failed) {
+                    st = BG_USER_ERROR;
+                } else if (lane_bit(low) && L.t < L.end) {  // rk.rs:414-416
+                    st = BG_MINIMUM_TIME_DELTA_EXCEEDED;
+                    if (accepted) --nacc;
+                } else if (lane_bit(at_end)) {
+                    // the iterator's next step() would return Done (rk.rs:362-364)
+                    st = BG_OK;
+                } else if (attempts >= cap) {
+                    st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
                 }
             }
-            if (prio_cutoff) {
-                if (__ballot(inst >= 0 && pos < prio_cutoff) != 0)
-                    __builtin_amdgcn_s_setprio(2);
-                else
-                    __builtin_amdgcn_s_setprio(0);
-            }
+            budget -= first_of(made, running);
+            if (budget == 0) budget = cap - wave_max_u32(inst >= 0 && st < 0 ? attempts : 0u);
         }
-        if (__ballot(inst >= 0) == 0) break;
-        // ---- attempts ------------------------------------------------------
-        const uint64_t active = __ballot(inst >= 0);
-        const int want = min((int)refill_min, __popcll(active));
-        int st = (inst >= 0 && L.t >= L.end) ? BG_OK : -1;  // Done before any step
-        for (;;) {
-            const uint64_t done = __ballot(inst >= 0 && st >= 0);
-            if (__popcll(done) >= want) break;
-            if (inst >= 0 && st < 0) st = rk_advance(L, attempts, cap, nacc, nrej);
+        take = inst >= 0 && st >= 0;
+        if (take) {
+            // an attempt that ended in a failure counts as neither
+            const uint32_t lost =
+                st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u;
+            rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, attempts - nacc - lost);
+            inst = kNoInstance;
         }
-        if (inst >= 0 && st >= 0) {
-            rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, nrej);
-            inst = kNeedWork;
-        }
+        if (drained) break;
+        const uint64_t need = ballot(take);
+        pos = next_position(counter, need, desc_at_use(dv)->n, drained);
     }
 }
 
@@ -158,84 +201,90 @@ __global__ void __launch_bounds__(256)
 // stop time and an accepted clamped step lands exactly on it.
 template <class RHS, class Tab>
 __global__ void __launch_bounds__(256)
-    rk_path_ensemble_kernel(const bg_ensemble_desc *dv, const bg_path_desc *__restrict__ pd,
+    rk_path_ensemble_kernel(const bg_ensemble_desc, const bg_path_desc pd,
                             uint32_t *__restrict__ counter) {
     constexpr int D = RHS::D;
     r8_init();
+    const karg_desc dv = kernarg_desc();
     RkLane<RHS, Tab> L;
-    const int lane = __lane_id();
-    const uint64_t max_att = dv->max_attempts;
-    const uint32_t cap = (uint32_t)((max_att && max_att < kDefaultMaxAttempts) ? max_att
-                                                                                : kDefaultMaxAttempts);
-    const uint32_t every = pd->every ? pd->every : 1u;
-    const uint32_t capacity = pd->capacity;
-    const bool stops_only = (pd->flags & BG_PATH_STOPS_ONLY) != 0;
-    const bool inst_major = (pd->flags & BG_PATH_INSTANCE_MAJOR) != 0;
+    const uint32_t cap = attempt_cap(dv->max_attempts);
+    const uint64_t n = dv->n;
+    const uint32_t every = pd.every ? pd.every : 1u;
+    const uint32_t capacity = pd.capacity;
+    const bool stops_only = (pd.flags & BG_PATH_STOPS_ONLY) != 0;
+    const bool inst_major = (pd.flags & BG_PATH_INSTANCE_MAJOR) != 0;
     // global-memory views: FLAT stores would make the next LDS read (the
     // root8 table) wait until they complete
-    const __attribute__((address_space(1))) double *stops = gptr(pd->stops);
-    __attribute__((address_space(1))) double *path_t = gptr(pd->path_t);
-    __attribute__((address_space(1))) double *path_y = gptr(pd->path_y);
-    __attribute__((address_space(1))) uint32_t *path_len = gptr(pd->path_len);
-    const uint32_t n_stops_all = pd->n_stops;
-    int64_t inst = kNeedWork;
-    uint32_t attempts = 0, nacc = 0, nrej = 0, next_stop = 0, n_stops = 0, nrec = 0;
+    const __attribute__((address_space(1))) double *stops = gptr(pd.stops);
+    __attribute__((address_space(1))) double *path_t = gptr(pd.path_t);
+    __attribute__((address_space(1))) double *path_y = gptr(pd.path_y);
+    const uint32_t n_stops_all = pd.n_stops;
+    uint32_t budget = cap;
+    bool drained = counter == nullptr;
+    int64_t inst = kNoInstance;
+    uint64_t pos = first_position();
+    bool take = true;
+    uint32_t attempts = 0, nacc = 0, next_stop = 0, n_stops = 0, nrec = 0;
     uint32_t every_left = every;  // accepted steps until the next record
     uint32_t slot = 0;            // ring entry of the next record (nrec % capacity)
     double target = 0.0;          // the next stop, else the end
     for (;;) {
-        const uint64_t need = __ballot(inst == kNeedWork);
-        if (need != 0) {
-            const int leader = __ffsll((unsigned long long)need) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(need));
-            base = __shfl(base, leader);
-            if (inst == kNeedWork) {
-                const uint64_t pos =
-                    (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane) - 1ull));
-                const bg_ensemble_desc di = desc_inputs(dv);
-                if (pos < di.n) {
-                    inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
-                    rk_load(L, di, (uint64_t)inst);
-                    attempts = nacc = nrej = next_stop = nrec = 0;
-                    every_left = every;
-                    slot = 0;
-                    n_stops = 0;
-                    while (n_stops < n_stops_all && stops[n_stops] < L.end) ++n_stops;
-                    while (next_stop < n_stops && stops[next_stop] <= L.t) ++next_stop;
-                    target = next_stop < n_stops ? stops[next_stop] : L.end;
-                } else {
-                    inst = kExhausted;
-                }
+        int st = -1;
+        if (take) {
+            const bg_ensemble_desc di = desc_inputs(dv);
+            inst = kNoInstance;
+            if (pos < di.n) {
+                inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
+                rk_load(L, di, (uint64_t)inst);
+                attempts = nacc = next_stop = nrec = 0;
+                every_left = every;
+                slot = 0;
+                n_stops = 0;
+                while (n_stops < n_stops_all && stops[n_stops] < L.end) ++n_stops;
+                while (next_stop < n_stops && stops[next_stop] <= L.t) ++next_stop;
+                target = next_stop < n_stops ? stops[next_stop] : L.end;
+                if (L.t >= L.end) st = BG_OK;
+                L.set_range(target);
+                L.head(target);
             }
         }
-        if (__ballot(inst >= 0) == 0) break;
-        int st = (inst >= 0 && L.t >= L.end) ? BG_OK : -1;
+        const int active = __popcll(ballot(inst >= 0));
+        if (active == 0) break;
+        const int want = drained ? active : 1;
         for (;;) {
-            if (__ballot(inst >= 0 && st >= 0) != 0) break;
+            const uint64_t running = ballot(inst >= 0 && st < 0);
+            if (active - __popcll(running) >= want) break;
+            uint32_t made = 0;
             if (inst >= 0 && st < 0) {
-                if (attempts >= cap) {
-                    st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
-                } else {
+                bool failed;
+                uint64_t at_end, fail, out;
+                do {
                     const bool to_stop = next_stop < n_stops;
-                    bool clamped;
-                    const int r = L.attempt_to(target, to_stop, clamped);
-                    ++attempts;
-                    if (r == STEP_ACCEPTED) {
+                    const double dt_proposed = L.dt;
+                    uint32_t step = 0;
+                    const bool accepted = L.attempt(failed, step);
+                    const bool at_stop = accepted && L.clamped && to_stop;
+                    // an accepted step cut short to land on a stop hands the
+                    // next attempt at least the step size proposed before the
+                    // cut: a stop just past an accepted time must not shrink
+                    // dt below dt_min and fail a solve that succeeds without
+                    // the stop
+                    if (at_stop) L.dt = fmax(L.dt, dt_proposed);
+                    const bool low = L.dt < L.dt_min && L.t < L.end;
+                    if (accepted && !low) {
                         ++nacc;
-                        bool at_stop = false;
-                        if (clamped && to_stop) {
+                        if (at_stop) {
                             L.t = target;
                             ++next_stop;
                             target = next_stop < n_stops ? stops[next_stop] : L.end;
-                            at_stop = true;
+                            L.set_range(target);
                         }
-                        const bool last = L.t >= L.end;
                         --every_left;
-                        const bool rec = stops_only ? (at_stop || last) : (every_left == 0);
+                        const bool rec =
+                            stops_only ? (at_stop || L.t >= L.end) : (every_left == 0);
                         if (every_left == 0) every_left = every;
                         if (rec) {
-                            const uint64_t n = desc_at_use(dv)->n, i = (uint64_t)inst;
+                            const uint64_t i = (uint64_t)inst;
                             if (capacity) {
                                 const uint64_t e = slot;
                                 if (inst_major) {
@@ -252,20 +301,38 @@ __global__ void __launch_bounds__(256)
                             }
                             ++nrec;
                         }
-                        if (last) st = BG_OK;
-                    } else if (r == STEP_REJECTED) {
-                        ++nrej;
-                    } else {
-                        st = r;
                     }
-                }
+                    L.head(target);
+                    ++made;
+                    at_end = ballot(L.t >= L.end);
+                    fail = ballot(low);
+                    out = at_end | fail;
+                    if constexpr (kRhsFails<RHS>) out |= ballot(failed);
+                } while (out == 0 && made < budget);
+                attempts += made;
+                if (failed)
+                    st = BG_USER_ERROR;
+                else if (lane_bit(fail))
+                    st = BG_MINIMUM_TIME_DELTA_EXCEEDED;
+                else if (lane_bit(at_end))
+                    st = BG_OK;
+                else if (attempts >= cap)
+                    st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
             }
+            budget -= first_of(made, running);
+            if (budget == 0) budget = cap - wave_max_u32(inst >= 0 && st < 0 ? attempts : 0u);
         }
-        if (inst >= 0 && st >= 0) {
-            rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, nrej);
-            if (path_len) path_len[inst] = nrec;
-            inst = kNeedWork;
+        take = inst >= 0 && st >= 0;
+        if (take) {
+            const uint32_t lost =
+                st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u;
+            rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, attempts - nacc - lost);
+            if (pd.path_len) gptr(pd.path_len)[inst] = nrec;
+            inst = kNoInstance;
         }
+        if (drained) break;
+        const uint64_t need = ballot(take);
+        pos = next_position(counter, need, n, drained);
     }
 }
 
@@ -276,9 +343,7 @@ __global__ void __launch_bounds__(64) rk_plain_kernel(const bg_ensemble_desc d, 
     if (threadIdx.x != 0) return;
     RkLane<RHS, Tab> L;
     const uint64_t i = d.order ? (uint64_t)d.order[k] : k;
-    const uint32_t cap =
-        (uint32_t)((d.max_attempts && d.max_attempts < kDefaultMaxAttempts) ? d.max_attempts
-                                                                           : kDefaultMaxAttempts);
+    const uint32_t cap = attempt_cap(d.max_attempts);
     rk_load(L, d, i);
     uint32_t attempts = 0;
     uint32_t nacc = 0, nrej = 0;
@@ -311,6 +376,7 @@ __global__ void __launch_bounds__(64)
         for (int k = 0; k < D; ++k) L.K[s][k] = st->K[s][k];
 #pragma unroll
     for (int k = 0; k < RHS::P; ++k) L.p[k] = st->p[k];
+    L.set_range(L.end);
     uint32_t attempts = (uint32_t)st->attempts;
     const uint32_t max_att = (uint32_t)st->max_attempts;
     uint32_t nacc = st->n_accepted, nrej = st->n_rejected, count = 0;
@@ -351,13 +417,10 @@ __global__ void __launch_bounds__(64)
     st->count = count;
 }
 
-// Work-queue reset and descriptor copy into the per-launch workspace
-// (a kernel rather than memset/memcpy so the launch sequence stays capturable).
-__global__ void rk_setup_kernel(uint32_t *counter, bg_ensemble_desc *dst, const bg_ensemble_desc d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *counter = 0u;
-        *dst = d;
-    }
+// Work-queue start: the lanes' own positions are taken (a kernel rather than
+// a memset so the launch sequence stays capturable).
+__global__ void rk_counter_kernel(uint32_t *counter, uint32_t lanes) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) *counter = lanes;
 }
 
 // ---------------------------------------------------------------------------
@@ -435,17 +498,18 @@ int rk_launch_ensemble(int method, int rhs, int semantics, const bg_ensemble_des
         uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
         const uint64_t need = (d.n + block - 1) / block;
         if (grid > need) grid = need;
-        // workspace: [0,256) work counter, [256, ...) descriptor copy
-        char *ws = (char *)ws_in;
-        if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, kLaunchWorkspaceBytes, stream));
-        uint32_t *counter = (uint32_t *)ws;
-        bg_ensemble_desc *ddesc = (bg_ensemble_desc *)(ws + 256);
-        rk_setup_kernel<<<1, 64, 0, stream>>>(counter, ddesc, d);
         const uint32_t refill_min = lc.refill_min ? lc.refill_min : 1u;
-        rk_ensemble_kernel<R, T>
-            <<<(uint32_t)grid, block, 0, stream>>>(ddesc, counter, refill_min, lc.prio_cutoff);
+        // a lane for every instance: no queue, no workspace
+        const bool queue = d.n > grid * block;
+        char *ws = (char *)ws_in;
+        if (queue) {
+            if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, kLaunchWorkspaceBytes, stream));
+            rk_counter_kernel<<<1, 64, 0, stream>>>((uint32_t *)ws, (uint32_t)(grid * block));
+        }
+        rk_ensemble_kernel<R, T><<<(uint32_t)grid, block, 0, stream>>>(
+            d, queue ? (uint32_t *)ws : nullptr, refill_min, lc.prio_cutoff);
         const hipError_t launched = hipGetLastError();
-        if (!ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
+        if (queue && !ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
         BG_HIP_CHECK(launched);
         return BG_OK;
     });
@@ -478,16 +542,6 @@ int rk_launch_path(int method, int rhs, int semantics, uint32_t dim, PathState *
     });
 }
 
-__global__ void rk_path_setup_kernel(uint32_t *counter, bg_ensemble_desc *dst,
-                                     const bg_ensemble_desc d, bg_path_desc *pdst,
-                                     const bg_path_desc p) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *counter = 0u;
-        *dst = d;
-        *pdst = p;
-    }
-}
-
 int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensemble_desc &d,
                             const bg_path_desc &p, hipStream_t stream) {
     return visit_rk(method, rhs, semantics, d.dim, [&](auto rtag, auto ttag) -> int {
@@ -506,17 +560,15 @@ int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensembl
         uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
         const uint64_t need = (d.n + 255) / 256;
         if (grid > need) grid = need;
-        // workspace: [0,256) counter, then the two descriptor copies
-        const size_t off_p = (256 + sizeof(bg_ensemble_desc) + 255) & ~(size_t)255;
-        char *ws = nullptr;
-        BG_HIP_CHECK(hipMallocAsync((void **)&ws, off_p + sizeof(bg_path_desc), stream));
-        uint32_t *counter = (uint32_t *)ws;
-        bg_ensemble_desc *ddesc = (bg_ensemble_desc *)(ws + 256);
-        bg_path_desc *pdesc = (bg_path_desc *)(ws + off_p);
-        rk_path_setup_kernel<<<1, 64, 0, stream>>>(counter, ddesc, d, pdesc, p);
-        rk_path_ensemble_kernel<R, T><<<(uint32_t)grid, 256, 0, stream>>>(ddesc, pdesc, counter);
+        const bool queue = d.n > grid * 256;
+        uint32_t *counter = nullptr;
+        if (queue) {
+            BG_HIP_CHECK(hipMallocAsync((void **)&counter, kLaunchWorkspaceBytes, stream));
+            rk_counter_kernel<<<1, 64, 0, stream>>>(counter, (uint32_t)(grid * 256));
+        }
+        rk_path_ensemble_kernel<R, T><<<(uint32_t)grid, 256, 0, stream>>>(d, p, counter);
         const hipError_t launched = hipGetLastError();
-        BG_HIP_CHECK(hipFreeAsync(ws, stream));
+        if (queue) BG_HIP_CHECK(hipFreeAsync(counter, stream));
         BG_HIP_CHECK(launched);
         return BG_OK;
     });
