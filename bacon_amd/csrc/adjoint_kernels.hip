@@ -103,9 +103,9 @@ __global__ void __launch_bounds__(256)
     __shared__ double obs_lds[OBS_LDS ? kObsLds : 1];
     const double *obs = stage_obs<OBS_LDS>(obs_lds, ad->obs_t, n_obs);
     RkLane<RHS, Tab> L;
-    int64_t inst = -1;
-    uint64_t k = first_position();
-    bool take = true, drained = ws.counters == nullptr;
+    WaveQueue queue(ws.counters);
+    int64_t inst = queue.start(n, d.order);
+    bool take = inst >= 0;
     uint32_t budget = kAdjMaxAttempts;
     uint32_t attempts = 0, nacc = 0, next_stop = 0, n_stops = 0, nck = 0;
     uint32_t ck_left = K;  // accepted steps until the next checkpoint
@@ -113,39 +113,36 @@ __global__ void __launch_bounds__(256)
     for (;;) {
         int st = -1;
         if (take) {
-            inst = -1;
-            if (k < n) {
-                inst = d.order ? (int64_t)gptr(d.order)[k] : (int64_t)k;
-                const uint64_t i = (uint64_t)inst;
+            const uint64_t i = (uint64_t)inst;
 #pragma unroll
-                for (int c = 0; c < D; ++c) L.y[c] = gptr(d.y0)[c * n + i];
+            for (int c = 0; c < D; ++c) L.y[c] = gptr(d.y0)[c * n + i];
 #pragma unroll
-                for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
-                L.t = d.t0 ? gptr(d.t0)[i] : d.t0_s;
-                L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
-                L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
-                L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
-                L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
-                L.dt = (L.dt_max + L.dt_min) * 0.5;
-                attempts = nacc = next_stop = 0;
-                ck_left = K;
-                n_stops = count_stops(obs, n_obs, L.end);
-                target = n_stops > 0 ? obs[0] : L.end;
-                // checkpoint 0: the initial state
-                double *ck0 = ws.ck + i * maxck * F;
-                ck0[0] = L.t;
-                ck0[1] = L.dt;
-                ck0[2] = 0.0;
+            for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
+            L.t = d.t0 ? gptr(d.t0)[i] : d.t0_s;
+            L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
+            L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
+            L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
+            L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
+            L.dt = (L.dt_max + L.dt_min) * 0.5;
+            attempts = nacc = next_stop = 0;
+            ck_left = K;
+            n_stops = count_stops(obs, n_obs, L.end);
+            target = n_stops > 0 ? obs[0] : L.end;
+            // checkpoint 0: the initial state
+            double *ck0 = ws.ck + i * maxck * F;
+            ck0[0] = L.t;
+            ck0[1] = L.dt;
+            ck0[2] = 0.0;
 #pragma unroll
-                for (int c = 0; c < D; ++c) ck0[3 + c] = L.y[c];
-                nck = 1;
-                if (L.t >= L.end) st = BG_OK;
-                L.set_range(target);
-                L.head(target);
-            }
+            for (int c = 0; c < D; ++c) ck0[3 + c] = L.y[c];
+            nck = 1;
+            if (L.t >= L.end) st = BG_OK;
+            L.set_range(target);
+            L.head(target);
         }
         const int active = __popcll(ballot(inst >= 0));
         if (active == 0) break;
+        const bool drained = queue.drained();
         const int want = drained ? active : 1;
         for (;;) {
             const uint64_t running = ballot(inst >= 0 && st < 0);
@@ -215,7 +212,9 @@ __global__ void __launch_bounds__(256)
                 else if (lane_bit(full) || attempts >= kAdjMaxAttempts)
                     st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
             }
-            budget -= first_of(made, running);
+            const uint32_t rounds = first_of(made, running);
+            queue.ticks += rounds;
+            budget -= rounds;
             if (budget == 0)
                 budget = kAdjMaxAttempts - wave_max_u32(inst >= 0 && st < 0 ? attempts : 0u);
         }
@@ -247,11 +246,12 @@ __global__ void __launch_bounds__(256)
                     (st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u);
                 d.counts[i] = cc;
             }
-            inst = -1;
         }
         if (drained) break;
-        const uint64_t need = ballot(take);
-        k = next_position(ws.counters, need, n, drained);
+        uint32_t pos;
+        const int64_t got = queue.next(ws.counters, (uint32_t)n, d.order, take, pos);
+        if (take) inst = got;
+        take = take && inst >= 0;
     }
 }
 
@@ -434,42 +434,41 @@ __global__ void __launch_bounds__(256)
             for (int c = 0; c < D; ++c) rn[c] = ws.res[(i * n_obs + (uint64_t)k) * D + c];
         }
     };
-    uint64_t k = first_position();
-    bool take = true, drained = ws.counters == nullptr;
+    WaveQueue queue(ws.counters);
+    inst = queue.start(n, ws.order_b);
+    bool take = inst >= 0;
     for (;;) {
         if (take) {
-            inst = -1;
-            if (k < n) {
-                inst = (int64_t)ws.order_b[k];
-                const uint64_t i = (uint64_t)inst;
+            const uint64_t i = (uint64_t)inst;
 #pragma unroll
-                for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
-                L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
-                L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
-                L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
-                L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
+            for (int c = 0; c < RHS::P; ++c) L.p[c] = gptr(d.params)[c * n + i];
+            L.end = d.t_end ? gptr(d.t_end)[i] : d.t_end_s;
+            L.tol = d.tol ? gptr(d.tol)[i] : d.tol_s;
+            L.dt_min = d.dt_min ? gptr(d.dt_min)[i] : d.dt_min_s;
+            L.dt_max = d.dt_max ? gptr(d.dt_max)[i] : d.dt_max_s;
 #pragma unroll
-                for (int c = 0; c < P; ++c) pb[c] = 0.0;
-                n_stops = count_stops(obs, n_obs, L.end);
-                const bool final_obs = n_stops < n_obs && obs[n_stops] == L.end;
+            for (int c = 0; c < P; ++c) pb[c] = 0.0;
+            n_stops = count_stops(obs, n_obs, L.end);
+            const bool final_obs = n_stops < n_obs && obs[n_stops] == L.end;
 #pragma unroll
-                for (int c = 0; c < D; ++c)
-                    lam[c] = final_obs ? 2.0 * ws.res[(i * n_obs + n_stops) * D + c] : 0.0;
-                const int fw = d.status ? gptr(d.status)[i] : BG_OK;
-                seg = fw == BG_OK ? (int)ws.nck[i] - 1 : -1;
-                load_res((int)n_stops - 1, i);
-                if (seg >= 0) {
-                    load_ck(seg, i);
-                    load_h(seg, i);
-                }
+            for (int c = 0; c < D; ++c)
+                lam[c] = final_obs ? 2.0 * ws.res[(i * n_obs + n_stops) * D + c] : 0.0;
+            const int fw = d.status ? gptr(d.status)[i] : BG_OK;
+            seg = fw == BG_OK ? (int)ws.nck[i] - 1 : -1;
+            load_res((int)n_stops - 1, i);
+            if (seg >= 0) {
+                load_ck(seg, i);
+                load_h(seg, i);
             }
         }
         const int active = __popcll(ballot(inst >= 0));
         if (active == 0) break;
+        const bool drained = queue.drained();
         const int want = drained ? active : 1;
         bool fin = false;
         for (;;) {
             if (__popcll(ballot(inst >= 0 && fin)) >= want) break;
+            queue.ticks += 16;  // a segment: about 16 replayed and reversed steps
             if (inst >= 0 && !fin) {
                 if (seg < 0) {
                     fin = true;
@@ -562,11 +561,12 @@ __global__ void __launch_bounds__(256)
                 for (int c = 0; c < RHS::P; ++c)
                     gptr(ad->grad_params)[c * n + i] = fw == BG_OK ? pb[c] : nan;
             }
-            inst = -1;
         }
         if (drained) break;
-        const uint64_t need = ballot(take);
-        k = next_position(ws.counters + 1, need, n, drained);
+        uint32_t pos;
+        const int64_t got = queue.next(ws.counters + 1, (uint32_t)n, ws.order_b, take, pos);
+        if (take) inst = got;
+        take = take && inst >= 0;
     }
 }
 

@@ -659,28 +659,94 @@ __device__ __forceinline__ bg_ensemble_desc desc_outputs(DP dv_) {
 // ---------------------------------------------------------------------------
 // The work queue of a persistent launch.  Lane g of the grid starts with
 // schedule position g; positions from the number of lanes on are handed out by
-// a counter that starts there (one atomicAdd per wave).  A launch whose
-// positions all have a lane passes no counter: nothing to set up before it,
-// and no wave asks for more.  Once a wave has been told that the positions are
-// used up it runs its remaining lanes to their ends without asking again, and
-// stores them together.
+// a counter that starts there.  A launch whose positions all have a lane passes
+// no counter: nothing to set up before it, and no wave asks for more.
+//
+// A wave claims a run of positions with one atomicAdd and hands them to its
+// lanes as they finish.  One atomicAdd per finished lane made the counter the
+// bottleneck of short instances: it serves one request per ~12 ns whatever the
+// chip computes (10^6 Lotka-Volterra solves of 350 attempts: 8.5 ms, 1.2 ms
+// of it arithmetic; with runs 2.4 ms).  Long instances want the opposite: a
+// position that waits in one wave's run is one that no other wave can start
+// (2^20 Lorenz-63 solves of 9,000 attempts on two waves per SIMD: 53 ms one at
+// a time, 55 ms in runs of up to 64).  So the length of a run follows the time
+// the last one took: doubled below 128 loop iterations, halved above 512 (all
+// of a few thousand waves claiming every 128 attempts, 50 us, keep the counter
+// busy less than half the time), and never more than a quarter to a half of the
+// wave's even share of what is left.  With a schedule the run's entries are
+// loaded when it is claimed, one per lane, so a refill does not wait for its
+// order[] entry.
+//
+// Every function is called by the whole wave.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t first_position() {
-    return (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-}
-// positions for the lanes of `need`; drained (wave-uniform) is set once the
-// counter has passed n
-__device__ __forceinline__ uint64_t next_position(uint32_t *counter, uint64_t need, uint64_t n,
-                                                  bool &drained) {
-    const int lane = __lane_id();
-    const int leader = __ffsll((unsigned long long)need) - 1;
-    const uint32_t cnt = (uint32_t)__popcll(need);
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, cnt);
-    base = first_of(base, need);
-    drained = (uint64_t)base + cnt >= n;
-    return (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane) - 1ull));
-}
+struct WaveQueue {
+    uint32_t base, end;   // unassigned positions of the claimed run
+    uint32_t first;       // position whose schedule entry lane 0 holds
+    int32_t entry;        // schedule entry of position first + lane
+    bool open;            // the counter may hold more
+    uint32_t run;         // length of the next run
+    uint32_t ticks;       // loop iterations since the last claim
+
+    __device__ __forceinline__ WaveQueue(const uint32_t *counter)
+        : base(0), end(0), first(0), entry(0), open(counter != nullptr), run(1), ticks(0) {}
+
+    __device__ __forceinline__ bool drained() const { return !open && base >= end; }
+
+    // the instance of the lane's own position, -1 if there is none
+    __device__ __forceinline__ int64_t start(uint64_t n, const int32_t *order) const {
+        const uint64_t pos = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        if (pos >= n) return -1;
+        return order ? (int64_t)gptr(order)[pos] : (int64_t)pos;
+    }
+
+    // the next instance for every lane that wants one, -1 if there is none;
+    // pos: its schedule position
+    __device__ __forceinline__ int64_t next(uint32_t *counter, uint32_t n, const int32_t *order,
+                                            bool want, uint32_t &pos) {
+        const uint32_t lane = __lane_id();
+        const uint64_t need = ballot(want);
+        const uint32_t cnt = (uint32_t)__popcll(need);
+        const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+        const uint32_t avail = end - base;
+        bool have = want && rank < avail;
+        pos = base + rank;
+        int32_t idx = order ? __shfl(entry, (int)((pos - first) & 63u)) : (int32_t)pos;
+        if (cnt <= avail) {
+            base += cnt;
+        } else if (open) {
+            const uint32_t lacking = cnt - avail;
+            const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+            const uint32_t left = n - (end ? end : waves << 6);
+            const uint32_t share = left >> (33 - __builtin_clz(waves));
+            if (ticks < 128u)
+                run = run < 64u ? 2u * run : 64u;
+            else if (ticks > 512u)
+                run = run > 1u ? run >> 1 : 1u;
+            ticks = 0;
+            uint32_t size = run < share ? run : share;
+            size = size < lacking ? lacking : size;
+            uint32_t b = 0;
+            if (lane == 0) b = atomicAdd(counter, size);
+            b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+            open = b < n && size < n - b;
+            b = b < n ? b : n;
+            end = open ? b + size : n;
+            first = b;
+            if (order) entry = b + lane < end ? gptr(order)[b + lane] : 0;
+            const uint32_t at = rank - avail;
+            const int32_t other = order ? __shfl(entry, (int)(at & 63u)) : (int32_t)(b + at);
+            if (want && rank >= avail) {
+                pos = b + at;
+                idx = other;
+                have = pos < end;
+            }
+            base = lacking < end - b ? b + lacking : end;
+        } else {
+            base = end;
+        }
+        return have ? (int64_t)idx : -1;
+    }
+};
 
 // The largest value over the wave's lanes, wave-uniform (every lane active).
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {

@@ -10,10 +10,10 @@
 //    lives in VGPRs for the whole solve;
 //  * inputs and outputs are structure-of-arrays in HBM ([component][n]);
 //  * the launch is persistent (grid = resident blocks); a wave refills its
-//    idle lanes from a global work counter with one atomicAdd per wave
-//    (ballot + popcount rank), so finished instances retire without
+//    idle lanes from runs of positions that it claims from a global counter
+//    (WaveQueue in bg_device.h), so finished instances retire without
 //    stalling the other lanes; an ensemble that fits the resident lanes needs
-//    no counter (first_position, next_position in bg_device.h);
+//    no counter;
 //  * an optional schedule permutation hands out instances longest-first.
 #include "bg_device.h"
 #include "bg_internal.h"
@@ -21,7 +21,6 @@
 namespace bg {
 
 static constexpr uint64_t kDefaultMaxAttempts = 10000000ull;
-static constexpr int64_t kNoInstance = -1;
 
 template <class T>
 struct Tag {
@@ -97,8 +96,8 @@ __device__ __forceinline__ int rk_advance(RkLane<RHS, Tab, H> &L, uint32_t &atte
     return -1;
 }
 
-// Persistent ensemble kernel.  Outer loop: refill idle lanes (one atomicAdd
-// per wave), store finished instances.  Inner loop: step attempts until at
+// Persistent ensemble kernel.  Outer loop: refill idle lanes, store
+// finished instances.  Inner loop: step attempts until at
 // least `refill_min` lanes of the wave have finished, or, once the queue is
 // used up, all have.  Waves holding an instance among the first `prio_cutoff`
 // schedule positions run at raised wave priority so the longest solves are
@@ -118,27 +117,22 @@ __global__ void __launch_bounds__(256)
     RkLane<RHS, Tab, true> L;
     const uint32_t cap = attempt_cap(dv->max_attempts);
     uint32_t budget = cap;  // attempts until a lane could reach the cap
-    bool drained = counter == nullptr;
-    int64_t inst = kNoInstance;
-    uint64_t pos = first_position();
-    bool take = true;
+    WaveQueue queue(counter);
+    uint32_t pos = blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t inst = queue.start(dv->n, dv->order);
+    bool take = inst >= 0;
     uint32_t attempts = 0, nacc = 0;
     for (;;) {
         // ---- refill --------------------------------------------------------
         int st = -1;  // running; >= 0: the instance's status
         if (take) {
-            const bg_ensemble_desc di = desc_inputs(dv);  // one batch of loads
-            inst = kNoInstance;
-            if (pos < di.n) {
-                inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
-                rk_load(L, di, (uint64_t)inst);
-                attempts = nacc = 0;
-                if (L.t >= L.end) st = BG_OK;  // Done before any step
-                L.head(L.end);
-            }
+            rk_load(L, desc_inputs(dv), (uint64_t)inst);  // one batch of loads
+            attempts = nacc = 0;
+            if (L.t >= L.end) st = BG_OK;  // Done before any step
+            L.head(L.end);
         }
         if (prio_cutoff) {
-            if (__ballot(inst >= 0 && pos < prio_cutoff) != 0)
+            if (ballot(inst >= 0 && pos < prio_cutoff) != 0)
                 __builtin_amdgcn_s_setprio(2);
             else
                 __builtin_amdgcn_s_setprio(0);
@@ -146,6 +140,7 @@ __global__ void __launch_bounds__(256)
         const int active = __popcll(ballot(inst >= 0));
         if (active == 0) break;
         // ---- attempts ------------------------------------------------------
+        const bool drained = queue.drained();
         const int want = drained ? active : min((int)refill_min, active);
         for (;;) {
             const uint64_t running = ballot(inst >= 0 && st < 0);
@@ -176,7 +171,9 @@ __global__ void __launch_bounds__(256)
                     st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
                 }
             }
-            budget -= first_of(made, running);
+            const uint32_t rounds = first_of(made, running);
+            queue.ticks += rounds;
+            budget -= rounds;
             if (budget == 0) budget = cap - wave_max_u32(inst >= 0 && st < 0 ? attempts : 0u);
         }
         take = inst >= 0 && st >= 0;
@@ -185,11 +182,12 @@ __global__ void __launch_bounds__(256)
             const uint32_t lost =
                 st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u;
             rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, attempts - nacc - lost);
-            inst = kNoInstance;
         }
         if (drained) break;
-        const uint64_t need = ballot(take);
-        pos = next_position(counter, need, desc_at_use(dv)->n, drained);
+        const karg_desc du = desc_at_use(dv);
+        const int64_t got = queue.next(counter, (uint32_t)du->n, du->order, take, pos);
+        if (take) inst = got;
+        take = take && inst >= 0;
     }
 }
 
@@ -220,10 +218,9 @@ __global__ void __launch_bounds__(256)
     __attribute__((address_space(1))) double *path_y = gptr(pd.path_y);
     const uint32_t n_stops_all = pd.n_stops;
     uint32_t budget = cap;
-    bool drained = counter == nullptr;
-    int64_t inst = kNoInstance;
-    uint64_t pos = first_position();
-    bool take = true;
+    WaveQueue queue(counter);
+    int64_t inst = queue.start(n, dv->order);
+    bool take = inst >= 0;
     uint32_t attempts = 0, nacc = 0, next_stop = 0, n_stops = 0, nrec = 0;
     uint32_t every_left = every;  // accepted steps until the next record
     uint32_t slot = 0;            // ring entry of the next record (nrec % capacity)
@@ -231,25 +228,21 @@ __global__ void __launch_bounds__(256)
     for (;;) {
         int st = -1;
         if (take) {
-            const bg_ensemble_desc di = desc_inputs(dv);
-            inst = kNoInstance;
-            if (pos < di.n) {
-                inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
-                rk_load(L, di, (uint64_t)inst);
-                attempts = nacc = next_stop = nrec = 0;
-                every_left = every;
-                slot = 0;
-                n_stops = 0;
-                while (n_stops < n_stops_all && stops[n_stops] < L.end) ++n_stops;
-                while (next_stop < n_stops && stops[next_stop] <= L.t) ++next_stop;
-                target = next_stop < n_stops ? stops[next_stop] : L.end;
-                if (L.t >= L.end) st = BG_OK;
-                L.set_range(target);
-                L.head(target);
-            }
+            rk_load(L, desc_inputs(dv), (uint64_t)inst);
+            attempts = nacc = next_stop = nrec = 0;
+            every_left = every;
+            slot = 0;
+            n_stops = 0;
+            while (n_stops < n_stops_all && stops[n_stops] < L.end) ++n_stops;
+            while (next_stop < n_stops && stops[next_stop] <= L.t) ++next_stop;
+            target = next_stop < n_stops ? stops[next_stop] : L.end;
+            if (L.t >= L.end) st = BG_OK;
+            L.set_range(target);
+            L.head(target);
         }
         const int active = __popcll(ballot(inst >= 0));
         if (active == 0) break;
+        const bool drained = queue.drained();
         const int want = drained ? active : 1;
         for (;;) {
             const uint64_t running = ballot(inst >= 0 && st < 0);
@@ -319,7 +312,9 @@ __global__ void __launch_bounds__(256)
                 else if (attempts >= cap)
                     st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
             }
-            budget -= first_of(made, running);
+            const uint32_t rounds = first_of(made, running);
+            queue.ticks += rounds;
+            budget -= rounds;
             if (budget == 0) budget = cap - wave_max_u32(inst >= 0 && st < 0 ? attempts : 0u);
         }
         take = inst >= 0 && st >= 0;
@@ -328,11 +323,12 @@ __global__ void __launch_bounds__(256)
                 st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u;
             rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, attempts - nacc - lost);
             if (pd.path_len) gptr(pd.path_len)[inst] = nrec;
-            inst = kNoInstance;
         }
         if (drained) break;
-        const uint64_t need = ballot(take);
-        pos = next_position(counter, need, n, drained);
+        uint32_t pos;
+        const int64_t got = queue.next(counter, (uint32_t)n, desc_at_use(dv)->order, take, pos);
+        if (take) inst = got;
+        take = take && inst >= 0;
     }
 }
 
@@ -493,7 +489,17 @@ int rk_launch_ensemble(int method, int rhs, int semantics, const bg_ensemble_des
         int per_cu = 0;
         BG_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, rk_ensemble_kernel<R, T>, (int)block, 0));
-        if (lc.blocks_per_cu && (int)lc.blocks_per_cu < per_cu) per_cu = (int)lc.blocks_per_cu;
+        // Default resident blocks.  Waves on a SIMD are served oldest first, so
+        // with more than two the youngest crawl (third wave: 2 us an attempt
+        // against the first one's 0.4) and end late with what they started
+        // early; fewer than two leave issue slots idle.  Two when the
+        // instances' end times or tolerances differ (2^20 Lorenz-63, longest
+        // first: 57 / 52 / 57 / 59 / 61 ms at 1 .. 5 blocks per CU), three when
+        // they do not, which also hides the refills of short instances (10^6
+        // Lotka-Volterra: 3.1 / 2.5 / 2.5 / 2.8 / 2.9 ms; 200,000 plain
+        // Lorenz-63: 5.1 / 4.9 / 4.6 / 5.3 / 5.5 ms).
+        const int want = lc.blocks_per_cu ? (int)lc.blocks_per_cu : (d.tol || d.t_end ? 2 : 3);
+        if (want < per_cu) per_cu = want;
         if (per_cu < 1) per_cu = 1;
         uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
         const uint64_t need = (d.n + block - 1) / block;
@@ -506,8 +512,16 @@ int rk_launch_ensemble(int method, int rhs, int semantics, const bg_ensemble_des
             if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, kLaunchWorkspaceBytes, stream));
             rk_counter_kernel<<<1, 64, 0, stream>>>((uint32_t *)ws, (uint32_t)(grid * block));
         }
+        // With a schedule the longest instances are the first ones, and the
+        // waves that hold them go first (the older waves do anyway; once they
+        // have finished theirs they give way to the younger ones that still
+        // have theirs to run): 52.5 -> 49.1 ms on the workload above with the
+        // first three quarters of the lanes' positions, 49.7 with all of them,
+        // 51.5 with half.
+        const uint32_t prio = lc.prio_cutoff ? lc.prio_cutoff
+                              : d.order && queue ? (uint32_t)(grid * block / 4 * 3) : 0u;
         rk_ensemble_kernel<R, T><<<(uint32_t)grid, block, 0, stream>>>(
-            d, queue ? (uint32_t *)ws : nullptr, refill_min, lc.prio_cutoff);
+            d, queue ? (uint32_t *)ws : nullptr, refill_min, prio);
         const hipError_t launched = hipGetLastError();
         if (queue && !ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
         BG_HIP_CHECK(launched);
