@@ -7,14 +7,14 @@
 // (19/270) / dt * |corrector - predictor|, an RK4 bootstrap of O - 1 steps
 // after every step-size change, and the yield bookkeeping of the iterator.
 //
-// One lane per instance, refilled from a global work counter like the RK
-// ensemble kernel.  The derivative deque holds at most O - 1 entries when the
-// predictor runs, so it lives in registers as a shift register (a push that
-// follows a full deque drops the oldest entry, which is the reference's
-// push_back + pop_front).  The value deque only matters through its length
-// here (final states, not the path).  Arithmetic follows the oracle's DEVICE
-// profile operation by operation (explicit fma, rootn() for the step-size
-// factor), so results are bit-identical to it.
+// One lane per instance, refilled like the RK ensemble kernel's.  The
+// derivative deque holds at most O - 1 entries when the predictor runs, so it
+// lives in registers as a shift register (a push that follows a full deque
+// drops the oldest entry, which is the reference's push_back + pop_front).
+// The value deque only matters through its length here (final states, not the
+// path).  Arithmetic follows the oracle's DEVICE profile operation by
+// operation (explicit fma, rootn() for the step-size factor), so results are
+// bit-identical to it.
 //
 // Semantics: as built, the derivative of the first Adams step after a
 // bootstrap never joins the deque (adams.rs:434-441 pushes the value only),
@@ -100,18 +100,55 @@ struct AdamsCoef<3> {
     }
 };
 
+// The coefficients through SGPR pairs (kc): at each use, or once for a loop.
+template <class C>
+struct CoefAtUse {
+    __device__ __forceinline__ double pred(int k) const { return kc(C::pred(k)); }
+    __device__ __forceinline__ double corr(int k) const { return kc(C::corr(k)); }
+};
+template <class C, int O>
+struct CoefOnce {
+    double p[O - 1], c[O];
+    __device__ __forceinline__ CoefOnce() {
+#pragma unroll
+        for (int k = 0; k < O - 1; ++k) p[k] = kc(C::pred(k));
+#pragma unroll
+        for (int k = 0; k < O; ++k) c[k] = kc(C::corr(k));
+    }
+    __device__ __forceinline__ double pred(int k) const { return p[k]; }
+    __device__ __forceinline__ double corr(int k) const { return c[k]; }
+};
+
 enum : int { ADAMS_YIELD = -1, ADAMS_REDO = -2, ADAMS_DONE = -3 };
 
 // PATH: also keep the values of the last bootstrap (the value deque's
 // entries, oldest first), which the yield_memory countdown of adams.rs:415-428
 // yields; `yitem` names what a yield returns: -1 the current (t, y), else
 // that entry.  Without PATH both are dead and compile away.
-template <class RHS, int O, bool AsBuilt, bool PATH = false>
+// COLD: the values that only a change of the step size looks at (tolerance,
+// step bounds, the state before the bootstrap) lie in LDS, one column of
+// kColdStride doubles apart per value, instead of registers: the ensemble
+// kernel then holds four waves per SIMD without spills (spilled, each change of
+// the step size waited for some fifty scratch reloads: 262,144 Lorenz-63
+// instances to t = 10 at tol 1e-6 took 12.8 ms instead of 7.9).
+constexpr int kColdStride = 256;
+template <class RHS, int O, bool AsBuilt, bool PATH = false, bool COLD = false>
 struct AdamsLane {
     static constexpr int D = RHS::D;
     using C = AdamsCoef<O>;
-    double t, dt, end, tol, dt_min, dt_max;
-    double y[D], save[D], impl[D];
+    static constexpr int kCold = 3 + D;
+    double t, dt, end;
+    double cold_reg[COLD ? 1 : kCold];
+    double *cold_lds;  // COLD: this lane's column
+    __device__ __forceinline__ double &cold(int k) {
+        if constexpr (COLD) return cold_lds[k * kColdStride];
+        else return cold_reg[k];
+    }
+    __device__ __forceinline__ double &tol() { return cold(0); }
+    __device__ __forceinline__ double &dt_min() { return cold(1); }
+    __device__ __forceinline__ double &dt_max() { return cold(2); }
+    __device__ __forceinline__ double &save(int c) { return cold(3 + c); }
+    double y[D], impl[D];
     double dq[O - 1][D];  // derivative history, oldest first (shift register)
     double vt[PATH ? O - 1 : 1], vy[PATH ? O - 1 : 1][D];  // value deque (PATH only)
     int vlen;             // length of the value deque
@@ -130,6 +167,22 @@ struct AdamsLane {
             for (int c = 0; c < D; ++c) dq[k][c] = dq[k + 1][c];
 #pragma unroll
         for (int c = 0; c < D; ++c) dq[O - 2][c] = v[c];
+    }
+    // a history whose oldest entry is dq[r] put in order (r differs by lane)
+    __device__ __forceinline__ void rotate_history(uint32_t r) {
+#pragma unroll
+        for (int by = 1; by < O - 1; by <<= 1) {
+            double m[O - 1][D];
+#pragma unroll
+            for (int k = 0; k < O - 1; ++k)
+#pragma unroll
+                for (int c = 0; c < D; ++c)
+                    m[k][c] = (r & (uint32_t)by) ? dq[(k + by) % (O - 1)][c] : dq[k][c];
+#pragma unroll
+            for (int k = 0; k < O - 1; ++k)
+#pragma unroll
+                for (int c = 0; c < D; ++c) dq[k][c] = m[k][c];
+        }
     }
     // value push at the full deque: push_back + pop_front, as for dq
     __device__ __forceinline__ void push_v() {
@@ -194,8 +247,8 @@ struct AdamsLane {
         return BG_OK;
     }
 
-    __device__ __forceinline__ double q_of(double error) const {
-        return rootn<O>(tol / (2.0 * error));
+    __device__ __forceinline__ double q_of(double error) {
+        return rootn<O>(tol() / (2.0 * error));
     }
 
     // One AdamsSolver::step (adams.rs:411-561)
@@ -219,37 +272,59 @@ struct AdamsLane {
             if (rc) return rc;
             return ADAMS_YIELD;
         }
-        if (vlen == 0) {  // adams.rs:453-464
+        return vlen == 0 ? bootstrap() : multistep(impl);
+    }
+
+    // adams.rs:453-464
+    __device__ __forceinline__ int bootstrap() {
 #pragma unroll
-            for (int c = 0; c < D; ++c) save[c] = y[c];
-            if (t + dt * (double)(O - 1) >= end) dt = (end - t) / (double)(O - 1);
-            const int rc = runge_kutta<O - 1>();
-            if (rc) return rc;
-            ym = O;
-            return ADAMS_REDO;
-        }
-        // adams.rs:466-486
-        double pr[D], co[D];
+        for (int c = 0; c < D; ++c) save(c) = y[c];
+        if (t + dt * (double)(O - 1) >= end) dt = (end - t) / (double)(O - 1);
+        const int rc = runge_kutta<O - 1>();
+        if (rc) return rc;
+        ym = O;
+        return ADAMS_REDO;
+    }
+
+    // Predictor and corrector (adams.rs:466-486) from the derivative history,
+    // whose oldest entry is dq[u] (u = 0 outside the ensemble kernel's ordinary
+    // steps): corrected value, the predicted point's derivative and the squared
+    // distance of the two values.  False if the right-hand side reports an
+    // error.
+    template <class CF>
+    __device__ __forceinline__ bool predict_correct(int u, const CF &cf, double (&co)[D],
+                                                    double (&im)[D], double &ss) const {
+        double pr[D];
 #pragma unroll
         for (int c = 0; c < D; ++c) {
-            double sc = dq[0][c] * kc(C::pred(O - 2));
+            double sc = dq[u][c] * cf.pred(O - 2);
 #pragma unroll
-            for (int i = 1; i < O - 1; ++i) sc = fma(dq[i][c], kc(C::pred(O - i - 2)), sc);
+            for (int i = 1; i < O - 1; ++i)
+                sc = fma(dq[(u + i) % (O - 1)][c], cf.pred(O - i - 2), sc);
             pr[c] = fma(sc, dt, y[c]);
         }
-        if (!f(t + dt, pr, impl)) return BG_USER_ERROR;
-        double ss = 0.0;
+        if (!f(t + dt, pr, im)) return false;
+        ss = 0.0;
 #pragma unroll
         for (int c = 0; c < D; ++c) {
-            double sc = impl[c] * kc(C::corr(0));
+            double sc = im[c] * cf.corr(0);
 #pragma unroll
-            for (int i = 0; i < O - 1; ++i) sc = fma(dq[i][c], kc(C::corr(O - i - 1)), sc);
+            for (int i = 0; i < O - 1; ++i)
+                sc = fma(dq[(u + i) % (O - 1)][c], cf.corr(O - i - 1), sc);
             co[c] = fma(sc, dt, y[c]);
             const double df = co[c] - pr[c];
             ss = c == 0 ? df * df : fma(df, df, ss);
         }
+        return true;
+    }
+
+    // The step from a full history (adams.rs:466-561); im: the derivative at
+    // the predicted point
+    __device__ __forceinline__ int multistep(double (&im)[D]) {
+        double co[D], ss;
+        if (!predict_correct(0, CoefAtUse<C>{}, co, im, ss)) return BG_USER_ERROR;
         const double error = (kc(19.0 / 270.0) / dt) * sqrt(ss);
-        if (error <= tol) {  // adams.rs:490-525
+        if (error <= tol()) {  // adams.rs:490-525
 #pragma unroll
             for (int c = 0; c < D; ++c) y[c] = co[c];
             t += dt;
@@ -257,14 +332,14 @@ struct AdamsLane {
                 ym -= 1;
                 return ADAMS_REDO;
             }
-            push_d(impl);  // with the value push: lengths stay O - 1
-            if (error < 0.1 * tol) {
+            push_d(im);  // with the value push: lengths stay O - 1
+            if (error < 0.1 * tol()) {
                 const double q = q_of(error);
                 if (q > 4.0)
                     dt *= 4.0;
                 else
                     dt *= q;
-                if (dt > dt_max) dt = dt_max;
+                if (dt > dt_max()) dt = dt_max();
                 vlen = 0;
             }
             return ADAMS_YIELD;
@@ -273,14 +348,14 @@ struct AdamsLane {
         if (ym == O) {  // adams.rs:531-536
             t -= dt * (double)(O - 1);
 #pragma unroll
-            for (int c = 0; c < D; ++c) y[c] = save[c];
+            for (int c = 0; c < D; ++c) y[c] = save(c);
         }
         const double q = q_of(error);  // adams.rs:538-556
         if (q < 0.1)
             dt *= 0.1;
         else
             dt *= q;
-        if (dt < dt_min) return BG_MINIMUM_TIME_DELTA_EXCEEDED;
+        if (dt < dt_min()) return BG_MINIMUM_TIME_DELTA_EXCEEDED;
         vlen = 0;
         return ADAMS_REDO;
     }
@@ -293,15 +368,17 @@ struct AdamsLane {
         for (int k = 0; k < RHS::P; ++k) p[k] = d.params[(uint64_t)k * n + i];
         t = d.t0 ? d.t0[i] : d.t0_s;
         end = d.t_end ? d.t_end[i] : d.t_end_s;
-        tol = d.tol ? d.tol[i] : d.tol_s;
-        dt_min = d.dt_min ? d.dt_min[i] : d.dt_min_s;
-        dt_max = d.dt_max ? d.dt_max[i] : d.dt_max_s;
-        dt = (dt_max + dt_min) * 0.5;  // adams.rs:288
+        const double lo = d.dt_min ? d.dt_min[i] : d.dt_min_s;
+        const double hi = d.dt_max ? d.dt_max[i] : d.dt_max_s;
+        tol() = d.tol ? d.tol[i] : d.tol_s;
+        dt_min() = lo;
+        dt_max() = hi;
+        dt = (hi + lo) * 0.5;  // adams.rs:288
         vlen = 0;
         ym = 0;
         n_rej = 0;
 #pragma unroll
-        for (int c = 0; c < D; ++c) save[c] = impl[c] = 0.0;
+        for (int c = 0; c < D; ++c) impl[c] = 0.0;
 #pragma unroll
         for (int k = 0; k < O - 1; ++k)
 #pragma unroll
@@ -309,57 +386,167 @@ struct AdamsLane {
     }
 };
 
+// ---------------------------------------------------------------------------
+// Persistent ensemble kernel.
+//
+// A lane's calls of step() are of two kinds: the ordinary predictor-corrector
+// step at an unchanged step size (98 % of them on Lorenz-63 at tol 1e-6), and
+// everything around a change of the step size: the exact error and the new
+// size, the RK4 bootstrap (four steps, 20 right-hand sides), its first
+// multistep, the yields of the bootstrap's values.  In a wave some lane is
+// nearly always at the second kind, so running both in each pass costs every
+// lane the bootstrap on most of its steps.  Here they are two phases:
+//   * the ordinary steps of all lanes, until half of the wave's lanes have
+//     met something else.  A lane commits its step if the squared error lies
+//     clearly between the two thresholds (error <= tol and not below
+//     0.1 tol, each with a margin of 1e-10, far above the rounding of the
+//     exact test), which needs neither the square root nor the divisions;
+//     any other lane leaves its state as it was and waits;
+//   * the calls of the waiting lanes, with the exact test, until most of
+//     them are back at ordinary steps.  A bootstrap's yields change nothing
+//     but the counters and are settled at once.
+// 262,144 Lorenz-63 instances, t in [0, 10], tol 1e-6: 41.4 -> 7.9 ms; 20,000 of
+// them 14.8 -> 2.6; 20,000 Lotka-Volterra at tol 1e-5 0.91 -> 0.33 ms.  Waiting
+// until a quarter (5/8) of the lanes are left at ordinary steps instead of half:
+// 9.6 (7.9), 3.0 (2.8) and 0.29 (0.36) ms.
+// ---------------------------------------------------------------------------
 template <class RHS, int O, bool AsBuilt>
-__global__ void __launch_bounds__(256)
-    adams_ensemble_kernel(const bg_ensemble_desc *dv, uint32_t *__restrict__ counter) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+    adams_ensemble_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter) {
     constexpr int D = RHS::D;
-    AdamsLane<RHS, O, AsBuilt> L;
-    const int lane = __lane_id();
+    constexpr uint32_t kRoundCalls = 2 * (O + 2);  // at most this many calls per slow round
+    const karg_desc dv = kernarg_desc();
+    AdamsLane<RHS, O, AsBuilt, false, true> L;
+    __shared__ double cold[L.kCold * kColdStride];
+    L.cold_lds = cold + threadIdx.x;
+    const CoefOnce<AdamsCoef<O>, O> cf;
     const uint64_t max_att = dv->max_attempts;
     const uint32_t cap =
         (uint32_t)((max_att && max_att < kAdamsDefaultMaxSteps) ? max_att : kAdamsDefaultMaxSteps);
-    int64_t inst = -1;  // -1 need work, -2 exhausted
-    uint32_t steps = 0, nacc = 0;
+    WaveQueue queue(counter);
+    int64_t inst = queue.start(dv->n, dv->order);
+    bool take = inst >= 0;
+    // calls so far: those that yielded (nacc) and those that did not
+    uint32_t nacc = 0, other = 0;
+    bool slow = false;          // waits for the second phase
+    double ss_lo = 0.0, ss_hi = 0.0;  // ordinary steps: ss_lo < ss < ss_hi
+    int32_t left = (int32_t)cap;      // passes before a lane could reach the cap
     for (;;) {
-        const uint64_t need = __ballot(inst == -1);
-        if (need != 0) {
-            const int leader = __ffsll((unsigned long long)need) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(need));
-            base = __shfl(base, leader);
-            if (inst == -1) {
-                const uint64_t pos =
-                    (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane) - 1ull));
-                const bg_ensemble_desc di = desc_inputs(dv);
-                if (pos < di.n) {
-                    inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
-                    L.load(di, (uint64_t)inst);
-                    steps = nacc = 0;
-                } else {
-                    inst = -2;
-                }
-            }
-        }
-        if (__ballot(inst >= 0) == 0) break;
         int st = -1;
+        if (take) {
+            L.load(desc_inputs(dv), (uint64_t)inst);
+            nacc = other = 0;
+            slow = true;
+        }
+        const int active = __popcll(ballot(inst >= 0));
+        if (active == 0) break;
+        const bool drained = queue.drained();
+        const int want = drained ? active : 1;
         for (;;) {
-            if (__ballot(inst >= 0 && st >= 0) != 0) break;
-            if (inst >= 0 && st < 0) {
-                if (steps >= cap) {
-                    st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
-                } else {
-                    ++steps;
-                    const int r = L.step();
-                    if (r == ADAMS_YIELD)
-                        ++nacc;
-                    else if (r == ADAMS_DONE)
-                        st = BG_OK;
-                    else if (r != ADAMS_REDO)
-                        st = r;
+            const int running = __popcll(ballot(inst >= 0 && st < 0));
+            if (active - running >= want) break;
+            // ---- ordinary steps: O - 1 of them a pass, so that every one
+            // finds its history in place (a commit overwrites the oldest entry
+            // instead of moving the others up)
+            bool fast = inst >= 0 && st < 0 && !slow;
+            const int stop_at = running / 2;
+            int32_t made = 0;
+            if (__popcll(ballot(fast)) > stop_at && left >= O - 1) {
+                const uint32_t before = nacc;
+                do {
+#pragma unroll
+                    for (int u = 0; u < O - 1; ++u) {
+                        // the lanes that wait compute along and keep nothing
+                        double co[D], im[D], ss;
+                        const double tn = L.t + L.dt;
+                        const bool ok = L.predict_correct(u, cf, co, im, ss);
+                        fast = fast & ok & (ss > ss_lo) & (ss < ss_hi) & !(tn >= L.end);
+                        if (fast) {
+                            L.t = tn;
+#pragma unroll
+                            for (int c = 0; c < D; ++c) {
+                                L.y[c] = co[c];
+                                L.dq[u][c] = im[c];
+                            }
+                            ++nacc;
+                        }
+                    }
+                    made += O - 1;
+                } while (__popcll(ballot(fast)) > stop_at && made + (O - 1) <= left);
+                L.rotate_history((nacc - before) % (uint32_t)(O - 1));
+            }
+            left -= made;
+            queue.ticks += (uint32_t)made + 4u;
+            slow = inst >= 0 && st < 0 && !fast;
+            if (left <= 0) {
+                left = (int32_t)(cap - wave_max_u32(inst >= 0 && st < 0 ? nacc + other : 0u));
+                // a lane near the cap: every lane's next call is an exact one
+                if (left <= 8 * (int32_t)kRoundCalls) slow = inst >= 0 && st < 0;
+            }
+            // ---- calls of the lanes that wait
+            const int waiting = __popcll(ballot(slow));
+            for (int round = 0; round < 8; ++round) {
+                left -= (int32_t)kRoundCalls;
+                if (slow) {
+                    int r = ADAMS_REDO;
+                    bool called = true;
+                    if (nacc + other >= cap) {
+                        st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
+                        called = false;
+                    } else if (L.t >= L.end) {
+                        r = ADAMS_DONE;
+                    } else if (L.t + L.dt >= L.end) {  // adams.rs:447-451
+                        L.dt = L.end - L.t;
+                        r = L.template runge_kutta<1>();
+                        if (r == BG_OK) r = ADAMS_YIELD;
+                    } else if (L.vlen != 0) {
+                        double im[D];
+                        r = L.multistep(im);
+                        // the first one after a bootstrap: the bootstrap's
+                        // yields follow (adams.rs:415-441), one call each
+                        if (r == ADAMS_REDO && L.ym == O - 1) {
+                            const uint32_t room = cap - 1u - (nacc + other);
+                            nacc += (uint32_t)O < room ? (uint32_t)O : room;
+                            L.ym = 0;
+                            if (!AsBuilt) L.push_d(im);
+                        }
+                    } else {
+                        called = false;
+                    }
+                    if (called) {
+                        if (r == ADAMS_YIELD)
+                            ++nacc;
+                        else
+                            ++other;
+                        if (r == ADAMS_DONE)
+                            st = BG_OK;
+                        else if (r != ADAMS_YIELD && r != ADAMS_REDO)
+                            st = r;
+                    }
                 }
+                const bool boot = slow && st < 0 && L.vlen == 0 && nacc + other < cap &&
+                                  !(L.t >= L.end) && !(L.t + L.dt >= L.end);
+                if (boot) {  // adams.rs:453-464
+                    const int r = L.bootstrap();
+                    ++other;
+                    if (r != ADAMS_REDO) st = r;
+                }
+                if (slow && (st >= 0 || (L.vlen != 0 && L.ym == 0 && L.t + L.dt < L.end))) {
+                    slow = false;
+                    // (tol / c)^2 and (0.1 tol / c)^2, c = (19/270) / dt
+                    const double c = kc(19.0 / 270.0) / L.dt;
+                    const double hi = L.tol() / c, lo = 0.1 * hi;
+                    ss_hi = hi * hi * (1.0 - 1e-10);
+                    ss_lo = lo * lo * (1.0 + 1e-10);
+                    // out of the range in which the margins hold: every step
+                    // by the exact test
+                    if (!(ss_lo > 1e-280 && ss_hi < 1e280)) ss_lo = __builtin_inf();
+                }
+                if (4 * __popcll(ballot(slow)) <= waiting) break;
             }
         }
-        if (inst >= 0 && st >= 0) {
+        take = inst >= 0 && st >= 0;
+        if (take) {
             const bg_ensemble_desc d = desc_outputs(dv);
             const uint64_t n = d.n, i = (uint64_t)inst;
             if (d.t_out) d.t_out[i] = L.t;
@@ -374,8 +561,13 @@ __global__ void __launch_bounds__(256)
                 cn.n_rejected = L.n_rej;
                 d.counts[i] = cn;
             }
-            inst = -1;
         }
+        if (drained) break;
+        const karg_desc du = desc_at_use(dv);
+        uint32_t pos;
+        const int64_t got = queue.next(counter, (uint32_t)du->n, du->order, take, pos);
+        if (take) inst = got;
+        take = take && inst >= 0;
     }
 }
 
@@ -394,9 +586,9 @@ __global__ void __launch_bounds__(64)
     L.t = st->t;
     L.dt = st->dt;
     L.end = st->end;
-    L.tol = st->tol;
-    L.dt_min = st->dt_min;
-    L.dt_max = st->dt_max;
+    L.tol() = st->tol;
+    L.dt_min() = st->dt_min;
+    L.dt_max() = st->dt_max;
     L.vlen = st->vlen;
     L.ym = st->ym;
     L.yitem = -1;
@@ -404,7 +596,7 @@ __global__ void __launch_bounds__(64)
 #pragma unroll
     for (int c = 0; c < D; ++c) {
         L.y[c] = st->y[c];
-        L.save[c] = st->save[c];
+        L.save(c) = st->save[c];
         L.impl[c] = st->impl[c];
     }
 #pragma unroll
@@ -462,7 +654,7 @@ __global__ void __launch_bounds__(64)
 #pragma unroll
     for (int c = 0; c < D; ++c) {
         st->y[c] = L.y[c];
-        st->save[c] = L.save[c];
+        st->save[c] = L.save(c);
         st->impl[c] = L.impl[c];
     }
 #pragma unroll
@@ -481,12 +673,8 @@ __global__ void __launch_bounds__(64)
     st->count = count;
 }
 
-__global__ void adams_setup_kernel(uint32_t *counter, bg_ensemble_desc *dst,
-                                   const bg_ensemble_desc d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *counter = 0u;
-        *dst = d;
-    }
+__global__ void adams_counter_kernel(uint32_t *counter, uint32_t lanes) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) *counter = lanes;
 }
 
 template <class T>
@@ -542,20 +730,21 @@ int adams_launch_ensemble(int method, int rhs, int semantics, const bg_ensemble_
         int per_cu = 0;
         BG_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, adams_ensemble_kernel<R, O, AB>, 256, 0));
-        // all resident blocks: 6 % faster than two per CU on 2^18 and 2^20
-        // Lorenz-63 instances (register-limited to 3 waves per SIMD)
         if (per_cu < 1) per_cu = 1;
         uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
         const uint64_t need = (d.n + 255) / 256;
         if (grid > need) grid = need;
+        // a lane for every instance: no queue, no workspace
+        const bool queue = d.n > grid * 256;
         char *ws = (char *)ws_in;
-        if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, kLaunchWorkspaceBytes, stream));
-        uint32_t *counter = (uint32_t *)ws;
-        bg_ensemble_desc *ddesc = (bg_ensemble_desc *)(ws + 256);
-        adams_setup_kernel<<<1, 64, 0, stream>>>(counter, ddesc, d);
-        adams_ensemble_kernel<R, O, AB><<<(uint32_t)grid, 256, 0, stream>>>(ddesc, counter);
+        if (queue) {
+            if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, kLaunchWorkspaceBytes, stream));
+            adams_counter_kernel<<<1, 64, 0, stream>>>((uint32_t *)ws, (uint32_t)(grid * 256));
+        }
+        adams_ensemble_kernel<R, O, AB><<<(uint32_t)grid, 256, 0, stream>>>(
+            d, queue ? (uint32_t *)ws : nullptr);
         const hipError_t launched = hipGetLastError();
-        if (!ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
+        if (queue && !ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
         BG_HIP_CHECK(launched);
         return BG_OK;
     });
