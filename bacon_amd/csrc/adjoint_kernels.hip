@@ -56,40 +56,6 @@ __global__ void adj_order_keys_kernel(const uint32_t *__restrict__ nck, uint64_t
     idx[i] = (int32_t)i;
 }
 
-// Observation times are read at every instance start (count_stops) and at
-// every stop.  With OBS_LDS (n_obs <= kObsLds) they are staged in LDS at
-// kernel entry: the reads then neither wait on L2 (a serial scan of 20
-// global loads per instance start cost microseconds) nor, being known LDS
-// accesses, wait for the loop's outstanding checkpoint stores.  Every thread
-// of the block calls it.
-static constexpr uint32_t kObsLds = 1024;
-template <bool OBS_LDS>
-__device__ __forceinline__ const double *stage_obs(double *lds, const double *obs,
-                                                   uint32_t n_obs) {
-    if constexpr (!OBS_LDS) {
-        return obs;
-    } else {
-        for (uint32_t k = threadIdx.x; k < n_obs; k += blockDim.x) lds[k] = gptr(obs)[k];
-        __syncthreads();
-        return lds;
-    }
-}
-
-// Number of observation times strictly before `end` (they become stops):
-// a binary search over the increasing times, ~log2(n_obs) dependent reads
-// at each instance start instead of one per time before the end.
-__device__ __forceinline__ uint32_t count_stops(const double *obs, uint32_t n_obs, double end) {
-    uint32_t lo = 0, hi = n_obs;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (obs[mid] < end)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 template <class RHS, class Tab, bool OBS_LDS>
 __global__ void __launch_bounds__(256)
     rk_adjoint_forward_kernel(const bg_adjoint_desc *__restrict__ ad, const AdjWs ws) {
@@ -102,6 +68,7 @@ __global__ void __launch_bounds__(256)
     const uint32_t n_obs = ad->n_obs;
     __shared__ double obs_lds[OBS_LDS ? kObsLds : 1];
     const double *obs = stage_obs<OBS_LDS>(obs_lds, ad->obs_t, n_obs);
+    const bool obs_mid = times_mid(obs, n_obs);
     RkLane<RHS, Tab> L;
     WaveQueue queue(ws.counters);
     int64_t inst = queue.start(n, d.order);
@@ -137,7 +104,7 @@ __global__ void __launch_bounds__(256)
             for (int c = 0; c < D; ++c) ck0[3 + c] = L.y[c];
             nck = 1;
             if (L.t >= L.end) st = BG_OK;
-            L.set_range(target);
+            L.set_range(obs_mid);
             L.head(target);
         }
         const int active = __popcll(ballot(inst >= 0));
@@ -176,7 +143,6 @@ __global__ void __launch_bounds__(256)
                                 ws.res[(i * n_obs + next_stop) * D + c] = L.y[c];
                             ++next_stop;
                             target = next_stop < n_stops ? obs[next_stop] : L.end;
-                            L.set_range(target);
                         }
                         --ck_left;
                         if (ck_left == 0 && !(L.t >= L.end)) {

@@ -340,6 +340,11 @@ __device__ __forceinline__ double qmin(double a, double b) {
     asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+__device__ __forceinline__ double qmax(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 __device__ __forceinline__ double qmax_one(double a) {
     double r;
     asm("v_max_f64 %0, %1, 1.0" : "=v"(r) : "v"(a));
@@ -450,13 +455,14 @@ struct RkLane {
         return kc(Tab::m(i, j));
     }
 
-    // Called when an instance is loaded and when the target changes: whether
-    // every quotient of the controller can take div_mid.  q2 = (tol h)^2 then
-    // lies in [2^-800, 2^800]: h is between dt_min and dt_max, or target - t,
-    // a multiple of 2^-153 unless the target lies within 2^-100 of zero.
-    __device__ __forceinline__ void set_range(double target) {
+    // Called when an instance is loaded: whether every quotient of the
+    // controller can take div_mid.  q2 = (tol h)^2 then lies in
+    // [2^-800, 2^800]: h is between dt_min and dt_max, or target - t, a
+    // multiple of 2^-153 unless the target (the end, or a stop: stops_mid)
+    // lies within 2^-100 of zero.
+    __device__ __forceinline__ void set_range(bool stops_mid = true) {
         const bool mid = tol >= 0x1p-200 && tol <= 0x1p200 && dt_min >= 0x1p-200 &&
-                         dt_max <= 0x1p200 && fabs(target) >= 0x1p-100;
+                         dt_max <= 0x1p200 && fabs(end) >= 0x1p-100 && stops_mid;
         r_lo = mid ? 1e-8 : __builtin_inf();
     }
 
@@ -747,6 +753,50 @@ struct WaveQueue {
         return have ? (int64_t)idx : -1;
     }
 };
+
+// ---------------------------------------------------------------------------
+// Shared stop (observation) times are read at every instance start
+// (count_stops) and at every stop.  With OBS_LDS (n_obs <= kObsLds) they are staged in LDS at
+// kernel entry: the reads then neither wait on L2 (a serial scan of 20
+// global loads per instance start cost microseconds) nor, being known LDS
+// accesses, wait for the loop's outstanding stores.  Every thread
+// of the block calls it.
+static constexpr uint32_t kObsLds = 1024;
+template <bool OBS_LDS>
+__device__ __forceinline__ const double *stage_obs(double *lds, const double *obs,
+                                                   uint32_t n_obs) {
+    if constexpr (!OBS_LDS) {
+        return obs;
+    } else {
+        for (uint32_t k = threadIdx.x; k < n_obs; k += blockDim.x) lds[k] = gptr(obs)[k];
+        __syncthreads();
+        return lds;
+    }
+}
+
+// Number of times strictly before `end` (those of them after the start become
+// stops): a binary search over the increasing times, ~log2(n_obs) dependent
+// reads at each instance start instead of one per time before the end.
+__device__ __forceinline__ uint32_t count_stops(const double *obs, uint32_t n_obs, double end) {
+    uint32_t lo = 0, hi = n_obs;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (obs[mid] < end)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// Whether no time lies within 2^-100 of zero (RkLane::set_range): increasing
+// times have at most one run of such values, around the first that is >= 0.
+__device__ __forceinline__ bool times_mid(const double *obs, uint32_t n_obs) {
+    const uint32_t k = count_stops(obs, n_obs, 0.0);
+    const bool above = k >= n_obs || obs[k] >= 0x1p-100;
+    const bool below = k == 0 || obs[k - 1] <= -0x1p-100;
+    return above && below;
+}
 
 // The largest value over the wave's lanes, wave-uniform (every lane active).
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {

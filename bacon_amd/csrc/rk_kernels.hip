@@ -51,7 +51,7 @@ __device__ __forceinline__ void rk_load(RkLane<RHS, Tab, H> &L, const bg_ensembl
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int k = 0; k < D; ++k) L.K[s][k] = 0.0;  // rk.rs:323-327
-    L.set_range(L.end);
+    L.set_range();
 }
 
 template <class RHS, class Tab, bool H>
@@ -191,53 +191,126 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Path output for an ensemble: the same persistent refill scheme as
+// Path output for an ensemble: the same persistent scheme as
 // rk_ensemble_kernel, and each accepted (t, y) the reference's IVPIterator
 // would yield (rk.rs:419, ivp.rs:220-238) is written to a per-instance ring
 // buffer: every `every`-th accepted step, or only landings on the shared stop
 // times and the end.  Stops: the end clamp of rk.rs:366-368 aims at the next
 // stop time and an accepted clamped step lands exactly on it.
-template <class RHS, class Tab>
+//
+// PACKED: records go to a workspace, [n][capacity][kRecord] doubles, and
+// path_unpack_kernel moves the ring's final content to the caller's arrays.
+// Instances drift apart by many steps, so in the caller's layouts an 8-byte
+// store is mostly alone in its cache line when the line leaves L2, and every
+// record costs 1 + D lines of traffic (262,144 Lorenz-63 instances, 524 M
+// records of 32 bytes: 134 GB of lines, 25-40 ms).  Packed, an instance fills
+// one line in four steps, and the lines that are open at a time (one per
+// resident lane, 3 MB per XCD) fit L2: 41 -> 8.5 ms, of which recording every
+// step takes 1.7 and the move 0.2; instance-major 17 -> 8.6.
+template <int D>
+constexpr int kRecord = (D + 2) / 2 * 2;  // t, y[D], padded to 16 bytes
+
+// Three loops, so that none carries the others' bookkeeping:
+//   kRing       no stops, records by count;
+//   kRingStops  stops between the records, or too many of them for LDS;
+//   kStopsOnly  records at stops and the end only, the stops in LDS.  In a wave
+//               of 64 lanes some lane lands on most attempts, so a landing is
+//               one branch: the stop after the one aimed at is read ahead.
+// The records' addresses advance with them, one per lane, the distances in
+// vector registers (the coefficients take the scalar ones).
+enum PathLoop { kRing, kRingStops, kStopsOnly };
+template <class RHS, class Tab, bool PACKED, PathLoop LOOP>
 __global__ void __launch_bounds__(256)
     rk_path_ensemble_kernel(const bg_ensemble_desc, const bg_path_desc pd,
-                            uint32_t *__restrict__ counter) {
+                            uint32_t *__restrict__ counter, double *records,
+                            uint32_t *__restrict__ n_records) {
     constexpr int D = RHS::D;
+    constexpr bool STOPS = LOOP != kRing;
     r8_init();
     const karg_desc dv = kernarg_desc();
-    RkLane<RHS, Tab> L;
+    RkLane<RHS, Tab, true> L;
     const uint32_t cap = attempt_cap(dv->max_attempts);
     const uint64_t n = dv->n;
     const uint32_t every = pd.every ? pd.every : 1u;
     const uint32_t capacity = pd.capacity;
     const bool stops_only = (pd.flags & BG_PATH_STOPS_ONLY) != 0;
     const bool inst_major = (pd.flags & BG_PATH_INSTANCE_MAJOR) != 0;
-    // global-memory views: FLAT stores would make the next LDS read (the
-    // root8 table) wait until they complete
-    const __attribute__((address_space(1))) double *stops = gptr(pd.stops);
-    __attribute__((address_space(1))) double *path_t = gptr(pd.path_t);
-    __attribute__((address_space(1))) double *path_y = gptr(pd.path_y);
-    const uint32_t n_stops_all = pd.n_stops;
+    uint64_t stride = inst_major ? 1u : n;  // between an entry's components
+    asm("" : "+v"(stride));
+    const uint32_t n_stops_all = STOPS ? pd.n_stops : 0u;
+    __shared__ double stops_lds[STOPS ? kObsLds : 1];
+    const bool in_lds = LOOP == kStopsOnly || n_stops_all <= kObsLds;
+    bool stops_mid = true;
+    if constexpr (STOPS) {
+        if (in_lds) stage_obs<true>(stops_lds, pd.stops, n_stops_all);
+        stops_mid = in_lds ? times_mid(stops_lds, n_stops_all) : times_mid(pd.stops, n_stops_all);
+    }
+    // the k-th time to aim at: a stop, else the end
+    auto aim = [&](uint32_t k, uint32_t count, double end) -> double {
+        if (!STOPS || k >= count) return end;
+        return in_lds ? stops_lds[k] : gptr(pd.stops)[k];
+    };
     uint32_t budget = cap;
     WaveQueue queue(counter);
     int64_t inst = queue.start(n, dv->order);
     bool take = inst >= 0;
     uint32_t attempts = 0, nacc = 0, next_stop = 0, n_stops = 0, nrec = 0;
     uint32_t every_left = every;  // accepted steps until the next record
-    uint32_t slot = 0;            // ring entry of the next record (nrec % capacity)
+    uint32_t room = 0;            // entries until the ring wraps
+    double *at_t = nullptr, *at_y = nullptr;  // the next record's place
     double target = 0.0;          // the next stop, else the end
+    double after = 0.0;           // the one after it
+    auto ring_start = [&]() {
+        const uint64_t i = (uint64_t)inst;
+        room = capacity;
+        if constexpr (PACKED) {
+            at_t = records + i * capacity * kRecord<D>;
+        } else {
+            at_t = pd.path_t + i * (inst_major ? capacity : 1u);
+            at_y = pd.path_y + i * (inst_major ? (uint64_t)capacity * D : 1u);
+        }
+    };
+    auto record = [&]() {
+        if (capacity) {
+            if constexpr (PACKED) {
+                typedef double pair_t __attribute__((ext_vector_type(2)));
+                auto *p = gptr((pair_t *)at_t);
+                p[0] = pair_t{L.t, L.y[0]};
+#pragma unroll
+                for (int c = 1; c < D; c += 2)
+                    p[(c + 1) / 2] = pair_t{L.y[c], L.y[c + 1 < D ? c + 1 : c]};
+                at_t += kRecord<D>;
+            } else {
+                *gptr(at_t) = L.t;
+                at_t += stride;
+#pragma unroll
+                for (int c = 0; c < D; ++c) {
+                    *gptr(at_y) = L.y[c];
+                    at_y += stride;
+                }
+            }
+            if (--room == 0) ring_start();
+        }
+        ++nrec;
+    };
     for (;;) {
         int st = -1;
         if (take) {
             rk_load(L, desc_inputs(dv), (uint64_t)inst);
-            attempts = nacc = next_stop = nrec = 0;
+            attempts = nacc = nrec = 0;
             every_left = every;
-            slot = 0;
-            n_stops = 0;
-            while (n_stops < n_stops_all && stops[n_stops] < L.end) ++n_stops;
-            while (next_stop < n_stops && stops[next_stop] <= L.t) ++next_stop;
-            target = next_stop < n_stops ? stops[next_stop] : L.end;
+            ring_start();
+            if constexpr (STOPS) {
+                n_stops = in_lds ? count_stops(stops_lds, n_stops_all, L.end)
+                                 : count_stops(pd.stops, n_stops_all, L.end);
+                next_stop = in_lds ? count_stops(stops_lds, n_stops, L.t)
+                                   : count_stops(pd.stops, n_stops, L.t);
+                while (next_stop < n_stops && aim(next_stop, n_stops, 0.0) <= L.t) ++next_stop;
+                after = aim(next_stop + 1, n_stops, L.end);
+            }
+            target = aim(next_stop, n_stops, L.end);
             if (L.t >= L.end) st = BG_OK;
-            L.set_range(target);
+            L.set_range(stops_mid);
             L.head(target);
         }
         const int active = __popcll(ballot(inst >= 0));
@@ -249,51 +322,46 @@ __global__ void __launch_bounds__(256)
             if (active - __popcll(running) >= want) break;
             uint32_t made = 0;
             if (inst >= 0 && st < 0) {
-                bool failed;
+                bool failed, accepted;
                 uint64_t at_end, fail, out;
                 do {
-                    const bool to_stop = next_stop < n_stops;
                     const double dt_proposed = L.dt;
-                    uint32_t step = 0;
-                    const bool accepted = L.attempt(failed, step);
-                    const bool at_stop = accepted && L.clamped && to_stop;
+                    accepted = L.attempt(failed, nacc);
+                    const bool at_stop =
+                        STOPS && accepted && L.clamped && next_stop < n_stops;
                     // an accepted step cut short to land on a stop hands the
                     // next attempt at least the step size proposed before the
                     // cut: a stop just past an accepted time must not shrink
                     // dt below dt_min and fail a solve that succeeds without
                     // the stop
-                    if (at_stop) L.dt = fmax(L.dt, dt_proposed);
+                    if constexpr (STOPS) {
+                        const double longer = qmax(L.dt, dt_proposed);
+                        L.dt = at_stop ? longer : L.dt;
+                    }
                     const bool low = L.dt < L.dt_min && L.t < L.end;
-                    if (accepted && !low) {
-                        ++nacc;
-                        if (at_stop) {
+                    if constexpr (LOOP == kStopsOnly) {
+                        if (accepted && !low && (at_stop || L.t >= L.end)) {
+                            const double read =
+                                stops_lds[next_stop + 2 < kObsLds ? next_stop + 2 : kObsLds - 1];
+                            const double later = next_stop + 2 < n_stops ? read : L.end;
+                            L.t = at_stop ? target : L.t;
+                            target = at_stop ? after : target;
+                            after = at_stop ? later : after;
+                            next_stop += at_stop ? 1u : 0u;
+                            record();
+                        }
+                    } else if (accepted && !low) {
+                        if (STOPS && at_stop) {
                             L.t = target;
                             ++next_stop;
-                            target = next_stop < n_stops ? stops[next_stop] : L.end;
-                            L.set_range(target);
+                            target = after;
+                            after = aim(next_stop + 1, n_stops, L.end);
                         }
                         --every_left;
-                        const bool rec =
-                            stops_only ? (at_stop || L.t >= L.end) : (every_left == 0);
+                        const bool rec = STOPS && stops_only ? (at_stop || L.t >= L.end)
+                                                             : (every_left == 0);
                         if (every_left == 0) every_left = every;
-                        if (rec) {
-                            const uint64_t i = (uint64_t)inst;
-                            if (capacity) {
-                                const uint64_t e = slot;
-                                if (inst_major) {
-                                    const uint64_t r = i * capacity + e;
-                                    path_t[r] = L.t;
-#pragma unroll
-                                    for (int c = 0; c < D; ++c) path_y[r * D + c] = L.y[c];
-                                } else {
-                                    path_t[e * n + i] = L.t;
-#pragma unroll
-                                    for (int c = 0; c < D; ++c) path_y[(e * D + c) * n + i] = L.y[c];
-                                }
-                                slot = slot + 1 == capacity ? 0u : slot + 1;
-                            }
-                            ++nrec;
-                        }
+                        if (rec) record();
                     }
                     L.head(target);
                     ++made;
@@ -303,14 +371,16 @@ __global__ void __launch_bounds__(256)
                     if constexpr (kRhsFails<RHS>) out |= ballot(failed);
                 } while (out == 0 && made < budget);
                 attempts += made;
-                if (failed)
+                if (failed) {
                     st = BG_USER_ERROR;
-                else if (lane_bit(fail))
+                } else if (lane_bit(fail)) {
                     st = BG_MINIMUM_TIME_DELTA_EXCEEDED;
-                else if (lane_bit(at_end))
+                    if (accepted) --nacc;
+                } else if (lane_bit(at_end)) {
                     st = BG_OK;
-                else if (attempts >= cap)
+                } else if (attempts >= cap) {
                     st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
+                }
             }
             const uint32_t rounds = first_of(made, running);
             queue.ticks += rounds;
@@ -323,12 +393,63 @@ __global__ void __launch_bounds__(256)
                 st == BG_USER_ERROR || st == BG_MINIMUM_TIME_DELTA_EXCEEDED ? 1u : 0u;
             rk_store(L, desc_outputs(dv), (uint64_t)inst, st, nacc, attempts - nacc - lost);
             if (pd.path_len) gptr(pd.path_len)[inst] = nrec;
+            if constexpr (PACKED) n_records[inst] = nrec;
         }
         if (drained) break;
         uint32_t pos;
         const int64_t got = queue.next(counter, (uint32_t)n, desc_at_use(dv)->order, take, pos);
         if (take) inst = got;
         take = take && inst >= 0;
+    }
+}
+
+// The packed records to the caller's arrays: only entries that were written
+// (the first min(records, capacity) of an instance).  A block moves
+// kUnpackSlots entries of 64 instances through LDS, so that it reads runs of
+// kUnpackSlots records and, in the default layout, writes 64 neighbours.
+// Bound by HBM: 537 MB in, 537 MB out in 0.21 ms (5.1 TB/s).
+constexpr int kUnpackSlots = 8;
+template <int D>
+__global__ void __launch_bounds__(256)
+    path_unpack_kernel(const double *__restrict__ records, const uint32_t *__restrict__ n_records,
+                       uint64_t n, const bg_path_desc pd) {
+    constexpr int W = kRecord<D>, RUN = kUnpackSlots * W;
+    __shared__ double tile[64][RUN + 1];
+    const uint32_t capacity = pd.capacity;
+    const uint64_t i0 = (uint64_t)blockIdx.x * 64;
+    const uint32_t e0 = blockIdx.y * kUnpackSlots;
+    const uint32_t slots = capacity - e0 < (uint32_t)kUnpackSlots ? capacity - e0 : kUnpackSlots;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t k = threadIdx.x; k < 64 * RUN; k += 256) {
+        const uint32_t i = k / RUN, f = k % RUN;
+        if (i0 + i < n && f < slots * W)
+            tile[i][f] = records[((i0 + i) * capacity + e0) * W + f];
+    }
+    __syncthreads();
+    if ((pd.flags & BG_PATH_INSTANCE_MAJOR) != 0) {
+        // consecutive threads: consecutive values of one instance
+        for (uint32_t k = threadIdx.x; k < 64u * kUnpackSlots * (1 + D); k += 256) {
+            const uint32_t i = k / (kUnpackSlots * (1 + D)), r = k % (kUnpackSlots * (1 + D));
+            const uint32_t e = r < kUnpackSlots ? r : (r - kUnpackSlots) / D;
+            if (i0 + i >= n || e >= slots || e0 + e >= n_records[i0 + i]) continue;
+            const uint64_t at = (i0 + i) * capacity + e0 + e;
+            if (r < kUnpackSlots) {
+                pd.path_t[at] = tile[i][e * W];
+            } else {
+                const uint32_t c = (r - kUnpackSlots) % D;
+                pd.path_y[at * D + c] = tile[i][e * W + 1 + c];
+            }
+        }
+    } else if (i0 + lane < n) {
+        const uint32_t have = n_records[i0 + lane];
+        for (uint32_t r = wave; r < slots * (1 + D); r += 4) {
+            const uint32_t e = r / (1 + D), c = r % (1 + D);
+            if (e0 + e >= have) break;
+            const uint64_t at = e0 + e;
+            const double v = tile[lane][e * W + c];
+            if (c == 0) pd.path_t[at * n + i0 + lane] = v;
+            else pd.path_y[(at * D + c - 1) * n + i0 + lane] = v;
+        }
     }
 }
 
@@ -372,7 +493,7 @@ __global__ void __launch_bounds__(64)
         for (int k = 0; k < D; ++k) L.K[s][k] = st->K[s][k];
 #pragma unroll
     for (int k = 0; k < RHS::P; ++k) L.p[k] = st->p[k];
-    L.set_range(L.end);
+    L.set_range();
     uint32_t attempts = (uint32_t)st->attempts;
     const uint32_t max_att = (uint32_t)st->max_attempts;
     uint32_t nacc = st->n_accepted, nrej = st->n_rejected, count = 0;
@@ -556,6 +677,9 @@ int rk_launch_path(int method, int rhs, int semantics, uint32_t dim, PathState *
     });
 }
 
+// Sizes between which the path kernel packs its records (see there).
+constexpr size_t kPackedMin = (size_t)32 << 20, kPackedMax = (size_t)8 << 30;
+
 int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensemble_desc &d,
                             const bg_path_desc &p, hipStream_t stream) {
     return visit_rk(method, rhs, semantics, d.dim, [&](auto rtag, auto ttag) -> int {
@@ -567,23 +691,73 @@ int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensembl
         if (p.n_stops && !p.stops) return BG_ERR_INVALID_ARGUMENT;
         int dev = 0;
         BG_HIP_CHECK(hipGetDevice(&dev));
-        int per_cu = 0;
-        BG_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, rk_path_ensemble_kernel<R, T>, 256, 0));
-        if (per_cu < 1) per_cu = 1;
-        uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
-        const uint64_t need = (d.n + 255) / 256;
-        if (grid > need) grid = need;
-        const bool queue = d.n > grid * 256;
-        uint32_t *counter = nullptr;
-        if (queue) {
-            BG_HIP_CHECK(hipMallocAsync((void **)&counter, kLaunchWorkspaceBytes, stream));
-            rk_counter_kernel<<<1, 64, 0, stream>>>(counter, (uint32_t)(grid * 256));
+        // Packed records when the caller's arrays are larger than the chip's
+        // L2 (below that the lines stay until they are full), unless only
+        // stops are recorded (there the lanes of a wave write the same entry
+        // within a short time), the instances' own lines of an instance-major
+        // array fit L2 (two per lane: 3.2 ms against 4.1 packed for 100,000
+        // instances and 1024 entries, 17.0 against 9.2 for 262,144 and 64) or
+        // the stream is being captured (the workspace is the size of the
+        // caller's arrays).
+        constexpr int W = kRecord<R::D>;
+        const size_t record_bytes = (size_t)d.n * p.capacity * W * sizeof(double);
+        double *records = nullptr;
+        uint32_t *n_records = nullptr;
+        bool pack = !(p.flags & BG_PATH_STOPS_ONLY) && record_bytes >= kPackedMin &&
+                    record_bytes <= kPackedMax &&
+                    !((p.flags & BG_PATH_INSTANCE_MAJOR) && d.n <= 131072);
+        if (pack) {
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            pack = hipStreamIsCapturing(stream, &capturing) == hipSuccess &&
+                   capturing == hipStreamCaptureStatusNone;
+            if (!pack) (void)hipGetLastError();
         }
-        rk_path_ensemble_kernel<R, T><<<(uint32_t)grid, 256, 0, stream>>>(d, p, counter);
-        const hipError_t launched = hipGetLastError();
-        if (queue) BG_HIP_CHECK(hipFreeAsync(counter, stream));
+        if (pack) {
+            const size_t bytes = record_bytes + d.n * sizeof(uint32_t);
+            if (hipMallocAsync((void **)&records, bytes, stream) != hipSuccess) {
+                (void)hipGetLastError();  // no room: straight to the caller's arrays
+                records = nullptr;
+            } else {
+                n_records = (uint32_t *)((char *)records + record_bytes);
+            }
+        }
+        const bool stops_only = (p.flags & BG_PATH_STOPS_ONLY) != 0;
+        const auto kern =
+            stops_only && p.n_stops <= kObsLds ? rk_path_ensemble_kernel<R, T, false, kStopsOnly>
+            : stops_only || p.n_stops > 0
+                ? (records ? rk_path_ensemble_kernel<R, T, true, kRingStops>
+                           : rk_path_ensemble_kernel<R, T, false, kRingStops>)
+                : (records ? rk_path_ensemble_kernel<R, T, true, kRing>
+                           : rk_path_ensemble_kernel<R, T, false, kRing>);
+        int per_cu = 0;
+        uint32_t *counter = nullptr;
+        auto run = [&]() -> hipError_t {
+            hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, 0);
+            if (e != hipSuccess) return e;
+            if (per_cu < 1) per_cu = 1;
+            uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
+            const uint64_t need = (d.n + 255) / 256;
+            if (grid > need) grid = need;
+            if (d.n > grid * 256) {
+                e = hipMallocAsync((void **)&counter, kLaunchWorkspaceBytes, stream);
+                if (e != hipSuccess) return e;
+                rk_counter_kernel<<<1, 64, 0, stream>>>(counter, (uint32_t)(grid * 256));
+            }
+            kern<<<(uint32_t)grid, 256, 0, stream>>>(d, p, counter, records, n_records);
+            if (records) {
+                const dim3 tiles((uint32_t)((d.n + 63) / 64),
+                                 (p.capacity + kUnpackSlots - 1) / kUnpackSlots);
+                path_unpack_kernel<R::D><<<tiles, 256, 0, stream>>>(records, n_records, d.n, p);
+            }
+            return hipGetLastError();
+        };
+        const hipError_t launched = run();
+        // the workspaces go back on every path
+        const hipError_t f1 = counter ? hipFreeAsync(counter, stream) : hipSuccess;
+        const hipError_t f2 = records ? hipFreeAsync(records, stream) : hipSuccess;
         BG_HIP_CHECK(launched);
+        BG_HIP_CHECK(f1);
+        BG_HIP_CHECK(f2);
         return BG_OK;
     });
 }
