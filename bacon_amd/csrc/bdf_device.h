@@ -52,33 +52,12 @@ __device__ __forceinline__ double dpp_f64(double v) {
         (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, false);
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
-// value of lane l ^ 16
-__device__ __forceinline__ uint32_t xor16_u32(uint32_t v) {
-    const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    return (__lane_id() & 16) ? p[0] : p[1];
-}
-__device__ __forceinline__ double xor16_f64(double v) {
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = xor16_u32((uint32_t)b), hi = xor16_u32((uint32_t)(b >> 32));
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 // value of lane l ^ 32, one 32-bit swap
 __device__ __forceinline__ float xor32_f32(float v) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     const auto p = __builtin_amdgcn_permlane32_swap(b, b, false, false);
     return __builtin_bit_cast(float, __lane_id() < 32 ? p[1] : p[0]);
 }
-// value of lane l ^ 32
-__device__ __forceinline__ double xor32_f64(double v) {
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
-    const auto hi =
-        __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
-    const bool low = __lane_id() < 32;
-    const uint32_t l = low ? lo[1] : lo[0], h = low ? hi[1] : hi[0];
-    return __builtin_bit_cast(double, ((uint64_t)h << 32) | l);
-}
-
 // lane l's value, broadcast (l wave-uniform)
 __device__ __forceinline__ double readlane_lu(double v, int l) {
     const uint64_t b = __builtin_bit_cast(uint64_t, v);

@@ -87,6 +87,7 @@ struct BogackiShampine23 {
 template <class Lit, bool AsBuilt>
 struct Tableau {
     static constexpr int S = Lit::S;
+    static constexpr bool as_built = AsBuilt;
     __host__ __device__ static constexpr double m(int i, int j) {
         return AsBuilt ? Lit::L[j][i] : Lit::L[i][j];
     }
@@ -357,6 +358,31 @@ __device__ __forceinline__ double qmin_s(double a, double b) {
     return r;
 }
 
+// Values of the lanes l ^ 16 and l ^ 32 by VALU lane swaps (gfx950):
+//   v_permlane16_swap(v, v): [0] = v[32 (l / 32) + l mod 16],
+//     [1] = v[32 (l / 32) + 16 + l mod 16]
+//   v_permlane32_swap(v, v): [0] = v[l mod 32], [1] = v[32 + l mod 32]
+// value of lane l ^ 16
+__device__ __forceinline__ uint32_t xor16_u32(uint32_t v) {
+    const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (__lane_id() & 16) ? p[0] : p[1];
+}
+__device__ __forceinline__ double xor16_f64(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = xor16_u32((uint32_t)b), hi = xor16_u32((uint32_t)(b >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// value of lane l ^ 32
+__device__ __forceinline__ double xor32_f64(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    const auto hi =
+        __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    const bool low = __lane_id() < 32;
+    const uint32_t l = low ? lo[1] : lo[0], h = low ? hi[1] : hi[0];
+    return __builtin_bit_cast(double, ((uint64_t)h << 32) | l);
+}
+
 // The lanes (of those active) for which c holds.
 __device__ __forceinline__ uint64_t ballot(bool c) { return __builtin_amdgcn_ballot_w64(c); }
 
@@ -380,6 +406,17 @@ __device__ __forceinline__ double div_mid(double a, double b) {
     const double y = fma(y0, fma(e, e, e), y0);
     const double q = a * y;
     return fma(fma(-b, q, a), y, q);
+}
+
+// The controller's factor before the tangent bound for a quotient r = q2 / ss
+// outside (r_lo, 65536), where the clamps delta <= 0.1 / delta >= 4 apply
+// (r <= 1e-8 / r >= 65536), the quotient needs the IEEE division (r_lo is +inf,
+// see RkLane::set_range) or it is NaN.  At 65536 and above only the quotient's
+// size matters.
+__device__ __forceinline__ double factor_outside(double q2, double ss, double r_lo, double &r) {
+    if (r >= 65536.0 && r_lo < 1.0) return 4.0;
+    r = q2 / ss;
+    return r <= 1e-8 ? 0.1 : (r >= 65536.0 ? 4.0 : root8(r));
 }
 
 // Right-hand sides that can report a UserError.
@@ -529,17 +566,6 @@ struct RkLane {
         if (!stages<false>(hh)) return false;
         update(hh);
         return true;
-    }
-
-    // The controller's factor for a quotient outside (r_lo, 65536), where the
-    // clamps delta <= 0.1 / delta >= 4 apply (r <= 1e-8 / r >= 65536), the
-    // quotient needs the IEEE division (see set_range) or it is NaN.  At
-    // 65536 and above only the quotient's size matters.
-    __device__ __forceinline__ static double factor_outside(double q2, double ss, double r_lo,
-                                                            double &r) {
-        if (r >= 65536.0 && r_lo < 1.0) return 4.0;
-        r = q2 / ss;
-        return r <= 1e-8 ? 0.1 : (r >= 65536.0 ? 4.0 : root8(r));
     }
 
     // One attempt of size h (head).  Returns whether it was accepted, and
