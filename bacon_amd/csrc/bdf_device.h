@@ -21,6 +21,7 @@
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "bg_device.h"
 #include "bg_internal.h"
@@ -90,12 +91,41 @@ __device__ __forceinline__ float pivot_recip(float a) {
 // ---------------------------------------------------------------------------
 // group collectives (every lane of the group active)
 // ---------------------------------------------------------------------------
+// value of the lane M apart (l ^ M), M = 1, 2, 4 or 8, by DPP moves
+template <int M>
+__device__ __forceinline__ double xor_f64(double v) {
+    if constexpr (M == 1) return dpp_f64<0xB1>(v);
+    else if constexpr (M == 2) return dpp_f64<0x4E>(v);
+    else if constexpr (M == 4) return dpp_f64<0x1B>(dpp_f64<0x141>(v));  // 7 - (l ^ 3)
+    else return dpp_f64<0x128>(v);  // rotation by 8 within 16
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+template <int M>
+__device__ __forceinline__ uint32_t xor_u32(uint32_t v) {
+    if constexpr (M == 1) return dpp_u32<0xB1>(v);
+    else if constexpr (M == 2) return dpp_u32<0x4E>(v);
+    else if constexpr (M == 4) return dpp_u32<0x1B>(dpp_u32<0x141>(v));
+    else return dpp_u32<0x128>(v);
+}
+
 template <int W>
 struct Grp {
     int g;  // lane index in the group
     __device__ __forceinline__ double bcast(double v, int src) const {
         if constexpr (W == 1) return v;
         return __shfl(v, src, W);
+    }
+    // lane K's value (K known at compile time: one DPP move per word where
+    // the group is within a quad)
+    template <int K>
+    __device__ __forceinline__ double bcast_at(double v) const {
+        if constexpr (W == 1) return v;
+        else if constexpr (W == 2) return dpp_f64<K | K << 2 | (2 + K) << 4 | (2 + K) << 6>(v);
+        else if constexpr (W == 4) return dpp_f64<K * 0x55>(v);
+        else return __shfl(v, K, W);
     }
     // all-reduce sum; symmetric pairings, so every lane gets the same bits
     __device__ __forceinline__ double sum(double v) const {
@@ -107,24 +137,27 @@ struct Grp {
             v += xor16_f64(v);
             return v;
         } else {
-#pragma unroll
-            for (int m = W / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, W);
+            if constexpr (W >= 16) v += xor_f64<8>(v);
+            if constexpr (W >= 8) v += xor_f64<4>(v);
+            if constexpr (W >= 4) v += xor_f64<2>(v);
+            if constexpr (W >= 2) v += xor_f64<1>(v);
             return v;
         }
     }
-    // all-reduce maximum of unsigned keys (W == 32: one DPP max per stage)
+    // all-reduce maximum of unsigned keys (one DPP max per stage)
     __device__ __forceinline__ uint32_t max_u32(uint32_t v) const {
         if constexpr (W == 32) {
-            v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));
-            v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));
-            v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));
-            v = __builtin_elementwise_max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));
+            v = __builtin_elementwise_max(v, dpp_u32<0xB1>(v));
+            v = __builtin_elementwise_max(v, dpp_u32<0x4E>(v));
+            v = __builtin_elementwise_max(v, dpp_u32<0x141>(v));
+            v = __builtin_elementwise_max(v, dpp_u32<0x140>(v));
             v = __builtin_elementwise_max(v, xor16_u32(v));
             return v;
         } else {
-#pragma unroll
-            for (int m = W / 2; m >= 1; m >>= 1)
-                v = __builtin_elementwise_max(v, (uint32_t)__shfl_xor((int)v, m, W));
+            if constexpr (W >= 16) v = __builtin_elementwise_max(v, xor_u32<8>(v));
+            if constexpr (W >= 8) v = __builtin_elementwise_max(v, xor_u32<4>(v));
+            if constexpr (W >= 4) v = __builtin_elementwise_max(v, xor_u32<2>(v));
+            if constexpr (W >= 2) v = __builtin_elementwise_max(v, xor_u32<1>(v));
             return v;
         }
     }
@@ -138,12 +171,32 @@ struct Grp {
             v = fmax(v, xor16_f64(v));
             return v;
         } else {
-#pragma unroll
-            for (int m = W / 2; m >= 1; m >>= 1) v = fmax(v, __shfl_xor(v, m, W));
+            if constexpr (W >= 16) v = fmax(v, xor_f64<8>(v));
+            if constexpr (W >= 8) v = fmax(v, xor_f64<4>(v));
+            if constexpr (W >= 4) v = fmax(v, xor_f64<2>(v));
+            if constexpr (W >= 2) v = fmax(v, xor_f64<1>(v));
             return v;
         }
     }
 };
+
+// sqrt(ss) <= bound (OR_EQUAL) or sqrt(ss) < bound, as the rounded square root
+// would decide.  SQUARES: away from the bound the squares decide (a margin of
+// 1e-10 each way, far above their rounding), within it the root itself.  Not
+// in the whole-wave solver, whose registers are full: there the branch cost
+// more in spills than the root (27.5 against 26.7 ms, 32,768 instances to t = 2).
+template <bool SQUARES, bool OR_EQUAL>
+__device__ __forceinline__ bool norm_below(double ss, double bound) {
+    if constexpr (SQUARES) {
+        const double b2 = bound * bound;
+        if (b2 > 1e-290) {
+            if (ss < b2 * (1.0 - 1e-10)) return true;
+            if (ss > b2 * (1.0 + 1e-10)) return false;
+        }
+    }
+    const double nrm = sqrt(ss);
+    return OR_EQUAL ? nrm <= bound : nrm < bound;
+}
 
 // maximum of unsigned keys over each 16-lane row (one DPP max per stage)
 __device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
@@ -226,6 +279,21 @@ struct RhsBrusselatorG {
             left = dpp_f64<0x121>(y);
             right = dpp_f64<0x12F>(y);
             other = xor16_f64(y);
+        } else if constexpr (CELLS == 8) {
+            // a species' 8 cells fill half a row: a rotation of the row, with
+            // the half's wrap from the rotation by 8 more
+            const double l1 = dpp_f64<0x121>(y), l9 = dpp_f64<0x129>(y);
+            const double r1 = dpp_f64<0x12F>(y), r9 = dpp_f64<0x127>(y);
+            left = c == 0 ? l9 : l1;
+            right = c == CELLS - 1 ? r9 : r1;
+            other = xor_f64<8>(y);
+        } else if constexpr (CELLS == 4) {
+            left = dpp_f64<0x93>(y);   // quad_perm [3, 0, 1, 2]
+            right = dpp_f64<0x39>(y);  // quad_perm [1, 2, 3, 0]
+            other = xor_f64<4>(y);
+        } else if constexpr (CELLS == 2) {
+            left = right = xor_f64<1>(y);
+            other = xor_f64<2>(y);
         } else {
             left = grp.bcast(y, base + (c + CELLS - 1) % CELLS);
             right = grp.bcast(y, base + (c + 1) % CELLS);
@@ -334,11 +402,15 @@ struct GatherBdf {
     static constexpr int D = R::D, P = R::P;
     static constexpr int W = D <= 1 ? 1 : D <= 2 ? 2 : D <= 4 ? 4 : D <= 8 ? 8 : D <= 16 ? 16 : 32;
     static_assert(D <= 16, "gathered systems take at most a 16-lane group");
+    template <class G, int... K>
+    __device__ __forceinline__ static void gather(double y, const G &grp, double (&yy)[D],
+                                                  std::integer_sequence<int, K...>) {
+        ((yy[K] = grp.template bcast_at<K>(y)), ...);
+    }
     template <class G>
     __device__ static bool lane_eval(double t, double y, const double *p, const G &grp, double &f) {
         double yy[D], ff[D];
-#pragma unroll
-        for (int k = 0; k < D; ++k) yy[k] = grp.bcast(y, k);
+        gather(y, grp, yy, std::make_integer_sequence<int, D>{});
         const bool ok = R::eval(t, yy, p, ff);
         f = 0.0;
 #pragma unroll
@@ -497,8 +569,23 @@ struct BdfLane {
         return true;
     }
 
-    // y_g = -(Jinv x)_g with x broadcast through LDS
+    // every component of x to every lane of a quad or pair
+    template <int... K>
+    __device__ __forceinline__ void spread(double x, double (&xs)[W],
+                                           std::integer_sequence<int, K...>) const {
+        ((xs[K] = grp.template bcast_at<K>(x)), ...);
+    }
+
+    // y_g = -(Jinv x)_g with x broadcast through LDS (quads: DPP moves)
     __device__ __forceinline__ double neg_jinv_times(double x) {
+        if constexpr (W <= 4) {
+            double xs[W];
+            spread(x, xs, std::make_integer_sequence<int, W>{});
+            double acc = 0.0;
+#pragma unroll
+            for (int j = 0; j < W; ++j) acc = fma(jinv[j], xs[j], acc);
+            return -acc;
+        }
         lds[grp.g] = x;
         __builtin_amdgcn_wave_barrier();
         double acc = 0.0;
@@ -621,33 +708,65 @@ struct BdfLane {
 #pragma unroll
         for (int j = 0; j < W; ++j) b[j] = (LuT)lds[grp.g * (W + 1) + j];
         __builtin_amdgcn_wave_barrier();
-        bool used = false, ok = true;
-        int my_col = 0;
+        return invert_row(b);
+    }
+
+    // The elimination on the rows in registers (b: row g).  The pivot row,
+    // scaled, goes to the other lanes through LDS, within a pair or quad by
+    // lane shuffles.  A padding row is its own column's pivot and changes no
+    // other row: its columns are not eliminated.
+    __device__ __forceinline__ bool invert_row(LuT (&b)[W]) {
+        bool used = grp.g >= D, ok = true;
+        int my_col = grp.g >= D ? grp.g : 0;
 #pragma unroll
-        for (int k = 0; k < W; ++k) {
+        for (int k = 0; k < D; ++k) {
             const double key = grp.max(pivot_key((double)b[k], !used, grp.g));
             if (!pivot_nonzero(key)) ok = false;
-            const bool piv = (pivot_lane(key) == grp.g);
+            const int pl = pivot_lane(key);
+            const bool piv = (pl == grp.g);
+            if constexpr (W == 1) {
+                b[0] = (LuT)1 / b[0];
+            } else if constexpr (W <= 4) {
+                const LuT ip = (LuT)1 / b[k];
+                const LuT f = b[k];
+                LuT pr[W];
+#pragma unroll
+                for (int j = 0; j < D; ++j) pr[j] = j == k ? ip : b[j] * ip;
+#pragma unroll
+                for (int j = 0; j < D; ++j) pr[j] = __shfl(pr[j], pl, W);
+#pragma unroll
+                for (int j = 0; j < D; ++j) {
+                    const LuT other = j == k ? -f * pr[k] : fma(-f, pr[j], b[j]);
+                    b[j] = piv ? pr[j] : other;
+                }
+            } else {
+                if (piv) {
+                    const LuT ip = (LuT)1 / b[k];
+#pragma unroll
+                    for (int j = 0; j < W; ++j)
+                        if (j != k) b[j] *= ip;
+                    b[k] = ip;
+#pragma unroll
+                    for (int j = 0; j < W; ++j) lds[j] = (double)b[j];
+                }
+                __builtin_amdgcn_wave_barrier();
+                if (!piv) {
+                    const LuT f = b[k];
+#pragma unroll
+                    for (int j = 0; j < W; ++j)
+                        if (j != k) b[j] = fma(-f, (LuT)lds[j], b[j]);
+                    b[k] = -f * (LuT)lds[k];
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
             if (piv) {
                 used = true;
                 my_col = k;
-                const LuT ip = (LuT)1 / b[k];
-#pragma unroll
-                for (int j = 0; j < W; ++j)
-                    if (j != k) b[j] *= ip;
-                b[k] = ip;
-#pragma unroll
-                for (int j = 0; j < W; ++j) lds[j] = (double)b[j];
             }
-            __builtin_amdgcn_wave_barrier();
-            if (!piv) {
-                const LuT f = b[k];
-#pragma unroll
-                for (int j = 0; j < W; ++j)
-                    if (j != k) b[j] = fma(-f, (LuT)lds[j], b[j]);
-                b[k] = -f * (LuT)lds[k];
-            }
-            __builtin_amdgcn_wave_barrier();
+        }
+        if constexpr (W == 1) {
+            jinv[0] = (double)b[0];
+            return ok;
         }
         // lane p: row col(p) of the inverse, column c belongs to inverse
         // column q with col(q) = c.  Scatter rows by col(), publish col() in
@@ -664,6 +783,53 @@ struct BdfLane {
         }
         __builtin_amdgcn_wave_barrier();
         return ok;
+    }
+
+    // The finite-difference Jacobian's right-hand sides (bdf.rs:396-406) for
+    // both of a step's secants: they start from the same guess at the same
+    // time, so the derivatives at the perturbed states are the same and only
+    // their combination with the history differs.  fx: own component of
+    // f(t, x + dt e_c) and f(t, x - dt e_c).
+    static constexpr bool kSharedFd = SPLIT == 1 && W <= 8;
+    struct FdPoints {
+        double f0, above[kSharedFd ? D : 1], below[kSharedFd ? D : 1];
+    };
+    __device__ __forceinline__ bool fd_points(double tt, FdPoints &fd) const {
+        double x = y;
+        if (!f(tt, x, fd.f0)) return false;
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+            const bool mine = (grp.g == c);
+            x = mine ? x + dt : x;
+            if (!f(tt, x, fd.above[c])) return false;
+            x = mine ? x - 2.0 * dt : x;
+            if (!f(tt, x, fd.below[c])) return false;
+            x = mine ? x + dt : x;
+        }
+        return true;
+    }
+    // Row g of the Jacobian from them; leaves the guess as the reference's
+    // column loop does.
+    template <bool LOWER>
+    __device__ __forceinline__ void fd_row(const FdPoints &fd, double denom, double &guess,
+                                           LuT (&b)[W]) const {
+        guess = y;
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+            const bool mine = (grp.g == c);
+            guess = mine ? guess + dt : guess;
+            const double above = combine<LOWER>(fd.above[c], guess);
+            guess = mine ? guess - 2.0 * dt : guess;
+            const double below = combine<LOWER>(fd.below[c], guess);
+            guess = mine ? guess + dt : guess;
+            b[c] = (LuT)((above + Sem::fd_sign * below) * denom);
+        }
+#pragma unroll
+        for (int c = D; c < W; ++c) b[c] = grp.g == c ? (LuT)1 : (LuT)0;
+        if (grp.g >= D) {
+#pragma unroll
+            for (int c = 0; c < D; ++c) b[c] = (LuT)0;
+        }
     }
 
     // bdf.rs:390-411 for the whole-wave layout (SPLIT = 2): the
@@ -906,17 +1072,27 @@ struct BdfLane {
 
     // bdf.rs:414-475; on success `guess` holds the corrected value.
     template <bool LOWER>
-    __device__ __forceinline__ int secant(double &guess) {
+    __device__ __forceinline__ int secant(const FdPoints &fd, double &guess) {
         const double tt = t + Sem::theta * dt;
         const double denom = 1.0 / (2.0 * dt);
         double F;
         guess = y;
-        double fx0;
-        if (!f(tt, guess, fx0)) return BG_USER_ERROR;
-        F = combine<LOWER>(fx0, guess);
-        if (!fd_jacobian<LOWER>(tt, denom, guess)) return BG_USER_ERROR;
-        ++n_lu;
-        if (!invert()) {
+        bool inverted;
+        if constexpr (kSharedFd) {
+            F = combine<LOWER>(fd.f0, guess);
+            LuT b[W];
+            fd_row<LOWER>(fd, denom, guess, b);
+            ++n_lu;
+            inverted = invert_row(b);
+        } else {
+            double fx0;
+            if (!f(tt, guess, fx0)) return BG_USER_ERROR;
+            F = combine<LOWER>(fx0, guess);
+            if (!fd_jacobian<LOWER>(tt, denom, guess)) return BG_USER_ERROR;
+            ++n_lu;
+            inverted = invert();
+        }
+        if (!inverted) {
             // bdf.rs:432-441: full-pivot LU, then QR, each on the Jacobian
             // rebuilt from the same evaluations
             if (!fd_jacobian<LOWER>(tt, denom, guess)) return BG_USER_ERROR;
@@ -949,12 +1125,19 @@ struct BdfLane {
                 for (int k = 0; k < W; ++k) u += lds[k * (W + 1) + grp.g];
             }
             __builtin_amdgcn_wave_barrier();
-            lds[grp.g] = u;
-            __builtin_amdgcn_wave_barrier();
             const double w = (s + adj) / pp;
+            if constexpr (W <= 4) {
+                double us[W];
+                spread(u, us, std::make_integer_sequence<int, W>{});
 #pragma unroll
-            for (int j = 0; j < WJ; ++j) jinv[j] = fma(lds[h * WJ + j], w, jinv[j]);
-            __builtin_amdgcn_wave_barrier();
+                for (int j = 0; j < W; ++j) jinv[j] = fma(us[j], w, jinv[j]);
+            } else {
+                lds[grp.g] = u;
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int j = 0; j < WJ; ++j) jinv[j] = fma(lds[h * WJ + j], w, jinv[j]);
+                __builtin_amdgcn_wave_barrier();
+            }
             // s = -Jinv_new F (bdf.rs:464-465) without a second product
             // through LDS: with Jinv_new = Jinv + w u^T and Jinv F = -adj - s
             // (the previous s was -Jinv F_l), -Jinv_new F = adj + s - w (u . F);
@@ -962,8 +1145,7 @@ struct BdfLane {
             const double uf = comp_sum(u * F);
             s = fma(-w, uf, adj + s);
             guess += s;
-            const double nrm = sqrt(comp_sum(s * s));
-            if (nrm <= tol) return BG_OK;
+            if (norm_below<SPLIT == 1, true>(comp_sum(s * s), tol)) return BG_OK;
         }
         return BG_MAXIMUM_ITERATIONS_EXCEEDED;
     }
@@ -1004,22 +1186,41 @@ struct BdfLane {
             *yv = y;
             return BDF_YIELD;
         }
-        if (!hist_full) {  // bdf.rs:537-546
-            save = y;
-            if (t + dt * (double)O >= end) dt = (end - t) / (double)O;
-            const int rc = runge_kutta<O, true>();
-            if (rc) return rc;
-            yield_memory = O + 1;
-            return BDF_REDO;
+        if (!hist_full) return bootstrap();
+        const int rc = multistep(rejected);
+        if (rc == BDF_YIELD) {
+            *yt = t;
+            *yv = y;
         }
-        double hi, lo;
-        int rc = secant<false>(hi);
+        return rc;
+    }
+
+    // bdf.rs:537-546
+    __device__ __forceinline__ int bootstrap() {
+        save = y;
+        if (t + dt * (double)O >= end) dt = (end - t) / (double)O;
+        const int rc = runge_kutta<O, true>();
         if (rc) return rc;
-        rc = secant<true>(lo);
+        yield_memory = O + 1;
+        return BDF_REDO;
+    }
+
+    // The step from a full history (bdf.rs:548-633); a yield is the current
+    // (t, y)
+    __device__ __forceinline__ int multistep(bool *rejected) {
+        *rejected = false;
+        double hi, lo;
+        FdPoints fd;
+        if constexpr (kSharedFd) {
+            if (!fd_points(t + Sem::theta * dt, fd)) return BG_USER_ERROR;
+        }
+        int rc = secant<false>(fd, hi);
+        if (rc) return rc;
+        rc = secant<true>(fd, lo);
         if (rc) return rc;
         const double dlt = hi - lo;
-        const double error = sqrt(grp.sum(dlt * dlt));
-        if (error <= tol) {  // bdf.rs:583-614
+        const double error2 = grp.sum(dlt * dlt);  // the squared error
+        if (norm_below<SPLIT == 1, true>(error2, tol)) {  // bdf.rs:583-614
             y = hi;
             t += dt;
             if (yield_memory == O + 1) {
@@ -1027,13 +1228,11 @@ struct BdfLane {
                 return BDF_REDO;
             }
             hist_shift(t, y);
-            if (error < 0.1 * tol) {
+            if (norm_below<SPLIT == 1, false>(error2, 0.1 * tol)) {
                 dt *= 2.0;
                 if (dt > dt_max) dt = dt_max;
                 hist_full = false;
             }
-            *yt = t;
-            *yv = y;
             return BDF_YIELD;
         }
         *rejected = true;
@@ -1074,85 +1273,183 @@ struct BdfLane {
 };
 
 // ---------------------------------------------------------------------------
-// persistent ensemble kernel: one instance per group, group refill
+// persistent ensemble kernels
 // ---------------------------------------------------------------------------
+// One instance per wave (the 32-component system).
 // Four waves per SIMD (the LDS limit): the solver is latency-bound (an LDS
 // round trip on every elimination step), and waves hide each other's
 // waits.  On the 32-component Brusselator, 4 waves with 101 VGPRs spilled
 // measured 392 ms against 395 ms for 3 waves with 43 spilled (FP32 inverse:
 // 240 against 248 ms); 3 had beaten 2 by 20 % before.
-template <class RHS, int O, class Sem, class LuT, int SPLIT>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
-    bdf_ensemble_kernel(const bg_ensemble_desc *dv, uint32_t *__restrict__ counter) {
+template <class RHS, int O, class Sem, class LuT, int WAVES>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
+    bdf_wave_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter) {
     constexpr int W = RHS::W;
-    constexpr int GW = W * SPLIT;  // lanes per instance
-    constexpr int GPW = 64 / GW;   // groups per wave
-    __shared__ double lds_all[GPW][W * (W + 1) + 2];
+    static_assert(W == 32, "a whole wave per instance");
+    __shared__ double lds_all[W * (W + 1) + 2];
+    const karg_desc dv = kernarg_desc();
     const int lane = __lane_id();
-    const int grp_id = lane / GW;
-    BdfLane<RHS, O, Sem, LuT, SPLIT> L;
+    BdfLane<RHS, O, Sem, LuT, 2> L;
     L.grp.g = lane % W;
-    L.h = (lane % GW) / W;
-    L.lds = lds_all[grp_id];
-    // one wave per block; SPLIT = 2 holds one instance per wave
-    if constexpr (SPLIT == 2 && sizeof(LuT) == sizeof(float)) {
+    L.h = lane / W;
+    L.lds = lds_all;
+    if constexpr (sizeof(LuT) == sizeof(float)) {
         __shared__ float prow_all[W];
         L.prow_f = prow_all;
     }
     const uint64_t max_att = dv->max_attempts;
     const uint32_t cap =
         (uint32_t)((max_att && max_att < kBdfDefaultMaxSteps) ? max_att : kBdfDefaultMaxSteps);
-    int64_t inst = -1;  // -1 need work, -2 exhausted
+    // schedule position: the wave's own first, then from the counter
+    uint32_t pos = blockIdx.x;
     for (;;) {
-        // group leaders that need work
-        const bool leader = (lane % GW == 0);
-        const uint64_t need = __ballot(leader && inst == -1);
-        if (need != 0) {
-            const int first = __ffsll((unsigned long long)need) - 1;
-            uint32_t base = 0;
-            if (lane == first) base = atomicAdd(counter, (uint32_t)__popcll(need));
-            base = __shfl(base, first);
-            // rank of my group's leader among needing leaders
-            const uint64_t below = need & ((1ull << (grp_id * GW)) - 1ull);
-            const bool my_need = (need >> (grp_id * GW)) & 1ull;
-            if (my_need) {
-                const uint64_t k = (uint64_t)base + (uint64_t)__popcll(below);
-                const bg_ensemble_desc di = desc_inputs(dv);
-                if (k < di.n) {
-                    inst = di.order ? (int64_t)di.order[k] : (int64_t)k;
-                    L.load(di, (uint64_t)inst);
-                } else {
-                    inst = -2;
-                }
+        const bg_ensemble_desc di = desc_inputs(dv);
+        if (pos >= di.n) break;
+        const uint64_t inst = di.order ? (uint64_t)di.order[pos] : (uint64_t)pos;
+        L.load(di, inst);
+        uint32_t steps = 0, nacc = 0, nrej = 0;
+        int st;
+        for (;;) {
+            if (steps >= cap) {
+                st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
+                break;
+            }
+            ++steps;
+            double yt, yv;
+            bool rej;
+            const int r = L.step(&yt, &yv, &rej);
+            if (rej) ++nrej;
+            if (r == BDF_YIELD) {
+                ++nacc;
+            } else if (r == BDF_DONE) {
+                st = BG_OK;
+                break;
+            } else if (r != BDF_REDO) {
+                st = r;
+                break;
             }
         }
-        if (__ballot(inst >= 0) == 0) break;
+        const bg_ensemble_desc d = desc_outputs(dv);
+        const uint64_t n = d.n, i = inst;
+        if (d.y_out && L.h == 0 && L.grp.g < RHS::D) d.y_out[(uint64_t)L.grp.g * n + i] = L.y;
+        if (lane == 0) {
+            if (d.t_out) d.t_out[i] = L.t;
+            if (d.status) d.status[i] = st;
+            if (d.counts) {
+                bg_counts c;
+                c.n_accepted = nacc;
+                c.n_rejected = nrej;
+                d.counts[i] = c;
+            }
+            if (d.work) {
+                bg_counts c;
+                c.n_accepted = L.n_newton;
+                c.n_rejected = L.n_lu;
+                d.work[i] = c;
+            }
+        }
+        if (counter == nullptr) break;
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(counter, 1u);
+        pos = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+    }
+}
+
+// One instance per group of W <= 16 lanes.
+// A wave alone on its SIMD is bound by its instruction count, so the group
+// collectives are DPP moves (a shuffle is two LDS-unit operations and a wait),
+// the finite differences' right-hand sides are evaluated once for both
+// secants, the bootstrap's yields are settled at once, and the groups take
+// their bootstraps before a multistep that all of them share.  Two waves per
+// SIMD are enough registers for the shared evaluations (four spilled them).
+// 16,384 Robertson instances, 405 yields each: 0.86 -> 0.39 ms; 131,072 3.07 ->
+// 1.85; Brusselator with 4 (8, 16) components, 8,192 instances, 0.74 -> 0.31
+// (1.04 -> 0.58, 2.40 -> 1.61); Lotka-Volterra 0.76 -> 0.35.
+template <class RHS, int O, class Sem, class LuT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8)))
+    bdf_ensemble_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter) {
+    constexpr int W = RHS::W;
+    constexpr int GPW = 64 / W;  // groups per wave
+    __shared__ double lds_all[GPW][W * (W + 1) + 2];
+    const karg_desc dv = kernarg_desc();
+    const int lane = __lane_id();
+    const int grp_id = lane / W;
+    BdfLane<RHS, O, Sem, LuT> L;
+    L.grp.g = lane % W;
+    L.lds = lds_all[grp_id];
+    const bool leader = (lane % W == 0);
+    const uint64_t max_att = dv->max_attempts;
+    const uint32_t cap =
+        (uint32_t)((max_att && max_att < kBdfDefaultMaxSteps) ? max_att : kBdfDefaultMaxSteps);
+    // schedule position: the group's own first, then from the counter (which
+    // starts behind the groups' own; none if every instance has a group)
+    uint64_t pos = (uint64_t)blockIdx.x * GPW + grp_id;
+    bool idle = false;  // this group has no further instance
+    for (;;) {
+        int64_t inst = -1;
+        if (!idle) {
+            const bg_ensemble_desc di = desc_inputs(dv);
+            if (pos < di.n) {
+                inst = di.order ? (int64_t)di.order[pos] : (int64_t)pos;
+                L.load(di, (uint64_t)inst);
+            } else {
+                idle = true;
+            }
+        }
         if (inst >= 0) {
+            // The groups of a wave go through the calls of step() together:
+            // first the final RK4 step or the bootstrap of those that are
+            // there, then the multistep of all that have a history, so a
+            // group that bootstraps takes its multistep in the same pass as
+            // the others.
             uint32_t steps = 0, nacc = 0, nrej = 0;
-            int st;
-            for (;;) {
+            int st = -1;
+            while (st < 0) {
+                int r = BDF_REDO;
+                bool called = false;
                 if (steps >= cap) {
                     st = BG_MAXIMUM_ITERATIONS_EXCEEDED;
-                    break;
-                }
-                ++steps;
-                double yt, yv;
-                bool rej;
-                const int r = L.step(&yt, &yv, &rej);
-                if (rej) ++nrej;
-                if (r == BDF_YIELD) {
-                    ++nacc;
-                } else if (r == BDF_DONE) {
+                } else if (L.t >= L.end) {
+                    ++steps;
                     st = BG_OK;
-                    break;
-                } else if (r != BDF_REDO) {
-                    st = r;
-                    break;
+                } else if (L.t + L.dt >= L.end) {  // bdf.rs:531-535
+                    ++steps;
+                    called = true;
+                    L.dt = L.end - L.t;
+                    r = L.template runge_kutta<1, false>();
+                    if (r == BG_OK) ++nacc;
+                    else st = r;
+                } else if (!L.hist_full) {
+                    ++steps;
+                    r = L.bootstrap();
+                    if (r != BDF_REDO) st = r;
+                }
+                if (st < 0 && !called && L.hist_full && steps < cap && !(L.t >= L.end) &&
+                    !(L.t + L.dt >= L.end)) {
+                    ++steps;
+                    bool rej;
+                    r = L.multistep(&rej);
+                    if (rej) ++nrej;
+                    if (r == BDF_YIELD) {
+                        ++nacc;
+                    } else if (r != BDF_REDO) {
+                        st = r;
+                    } else if (L.yield_memory == O) {
+                        // the first step after a bootstrap: the bootstrap's
+                        // values and this one are yielded next, one call each
+                        // (bdf.rs:500-525), which moves nothing but the history
+                        const uint32_t room = cap - steps;
+                        const uint32_t k = (uint32_t)O + 1u < room ? (uint32_t)O + 1u : room;
+                        steps += k;
+                        nacc += k;
+                        L.yield_memory = 0;
+                        L.hist_shift(L.t, L.y);
+                    }
                 }
             }
             const bg_ensemble_desc d = desc_outputs(dv);
             const uint64_t n = d.n, i = (uint64_t)inst;
-            if (d.y_out && L.h == 0 && L.grp.g < RHS::D) d.y_out[(uint64_t)L.grp.g * n + i] = L.y;
+            if (d.y_out && L.grp.g < RHS::D) d.y_out[(uint64_t)L.grp.g * n + i] = L.y;
             if (leader) {
                 if (d.t_out) d.t_out[i] = L.t;
                 if (d.status) d.status[i] = st;
@@ -1169,8 +1466,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
                     d.work[i] = c;
                 }
             }
-            inst = -1;
         }
+        if (counter == nullptr) break;
+        const uint64_t need = ballot(leader && !idle);
+        if (need == 0) break;
+        const int first = __ffsll((unsigned long long)need) - 1;
+        uint32_t base = 0;
+        if (lane == first) base = atomicAdd(counter, (uint32_t)__popcll(need));
+        base = first_of(base, need);
+        // rank of my group's leader among the leaders that ask
+        pos = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << (grp_id * W)) - 1ull));
     }
 }
 
@@ -1256,11 +1561,8 @@ __global__ void __launch_bounds__(64)
 }
 
 template <int = 0>
-__global__ void bdf_setup_kernel(uint32_t *counter, bg_ensemble_desc *dst, const bg_ensemble_desc d) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *counter = 0u;
-        *dst = d;
-    }
+__global__ void bdf_counter_kernel(uint32_t *counter, uint32_t groups) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) *counter = groups;
 }
 
 // ---------------------------------------------------------------------------
@@ -1326,12 +1628,22 @@ struct BTag {
     using type = T;
 };
 
+// few: the ensemble has at most three waves per SIMD, so the kernel that is
+// limited to three (and spills less) fits it: 100 (1000, 2000) Brusselator
+// instances to t = 1 1.04 -> 0.95 (1.50 -> 1.46, 2.00 -> 1.94) ms.
+template <class R, int O, class S, class F>
+static constexpr auto bdf_kernel(bool few) {
+    if constexpr (R::W == 32)
+        return few ? bdf_wave_kernel<R, O, S, F, 3> : bdf_wave_kernel<R, O, S, F, 4>;
+    else return bdf_ensemble_kernel<R, O, S, F>;
+}
+
 // Persistent grid (one wave per block, as many as are resident, at most
 // cap_per_cu per CU when cap_per_cu > 0) and the launch workspace: the work
-// counter and the descriptor copy.  *occupancy, if given, receives the
+// counter.  *occupancy, if given, receives the
 // resident blocks per CU before the cap.
 template <class R, int O, class S, class F>
-static int bdf_launch_shape(const bg_ensemble_desc &d, uint64_t &grid, size_t &bytes,
+static int bdf_launch_shape(const bg_ensemble_desc &d, uint64_t &grid, size_t &bytes, bool &few,
                             uint32_t cap_per_cu = 0, int *occupancy = nullptr) {
     constexpr int W = R::W;
     constexpr int SP = W == 32 ? 2 : 1;  // a 32-component instance takes the whole wave
@@ -1339,8 +1651,9 @@ static int bdf_launch_shape(const bg_ensemble_desc &d, uint64_t &grid, size_t &b
     int dev = 0;
     BG_HIP_CHECK(hipGetDevice(&dev));
     int per_cu = 0;
+    few = d.n <= (uint64_t)(12 * device_cu_count(dev));
     BG_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, bdf_ensemble_kernel<R, O, S, F, SP>, 64, 0));
+        &per_cu, bdf_kernel<R, O, S, F>(few), 64, 0));
     if (occupancy) *occupancy = per_cu;
     if (cap_per_cu && (int)cap_per_cu < per_cu) per_cu = (int)cap_per_cu;
     if (per_cu < 1) per_cu = 1;
@@ -1360,17 +1673,22 @@ static int bdf_launch_one(const bg_ensemble_desc &d, hipStream_t stream, void *w
     constexpr int SP = R::W == 32 ? 2 : 1;
     uint64_t grid = 0;
     size_t bytes = 0;
-    const int rc = bdf_launch_shape<R, O, S, F>(d, grid, bytes, cap_per_cu);
+    bool few = false;
+    const int rc = bdf_launch_shape<R, O, S, F>(d, grid, bytes, few, cap_per_cu);
     if (rc != BG_OK) return rc;
     if (ws_in && ws_bytes < bytes) return BG_ERR_INVALID_ARGUMENT;
+    // a group for every instance: no queue, no workspace
+    constexpr int GPW = 64 / (R::W * SP);
+    const bool queue = d.n > grid * GPW;
     char *ws = (char *)ws_in;
-    if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, bytes, stream));
-    uint32_t *counter = (uint32_t *)ws;
-    bg_ensemble_desc *ddesc = (bg_ensemble_desc *)(ws + 256);
-    bdf_setup_kernel<<<1, 64, 0, stream>>>(counter, ddesc, d);
-    bdf_ensemble_kernel<R, O, S, F, SP><<<(uint32_t)grid, 64, 0, stream>>>(ddesc, counter);
+    if (queue) {
+        if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, bytes, stream));
+        bdf_counter_kernel<<<1, 64, 0, stream>>>((uint32_t *)ws, (uint32_t)(grid * GPW));
+    }
+    bdf_kernel<R, O, S, F>(few)<<<(uint32_t)grid, 64, 0, stream>>>(
+        d, queue ? (uint32_t *)ws : nullptr);
     const hipError_t launched = hipGetLastError();
-    if (!ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
+    if (queue && !ws_in) BG_HIP_CHECK(hipFreeAsync(ws, stream));
     BG_HIP_CHECK(launched);
     return BG_OK;
 }

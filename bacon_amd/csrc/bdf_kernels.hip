@@ -57,7 +57,8 @@ int bdf_workspace_bytes(int method, int rhs, int semantics, int lu_fp32, const b
                                  using F = typename decltype(ftag)::type;
                                  constexpr int O = decltype(otag)::value;
                                  uint64_t grid = 0;
-                                 return bdf_launch_shape<R, O, S, F>(d, grid, *bytes, 0,
+                                 bool few = false;
+                                 return bdf_launch_shape<R, O, S, F>(d, grid, *bytes, few, 0,
                                                                      occupancy);
                              });
     if (rc != BG_ERR_UNSUPPORTED) return rc;

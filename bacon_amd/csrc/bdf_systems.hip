@@ -51,7 +51,8 @@ int bdf_sys_workspace_bytes(int method, int rhs, int semantics, int, const bg_en
         using S = typename decltype(stag)::type;
         constexpr int O = decltype(otag)::value;
         uint64_t grid = 0;
-        return bdf_launch_shape<R, O, S, double>(d, grid, *bytes, 0, occupancy);
+        bool few = false;
+        return bdf_launch_shape<R, O, S, double>(d, grid, *bytes, few, 0, occupancy);
     });
 }
 
