@@ -117,3 +117,20 @@ def test_quotients_outside_the_root(gpu, orc, case, method, semantics):
         w.update(tol=np.geomspace(1e60, 1e140, 300))
     g = _solve(w, method=getattr(L, method), max_attempts=cap, semantics=semantics)
     _same(w, g, getattr(O, method), cap, semantics)
+
+
+@pytest.mark.parametrize("fields", ["equal", "tol", "t_end", "all"])
+@pytest.mark.parametrize("n", [1, 2, 257, 4099])
+def test_builder_schedules(gpu, orc, n, fields):
+    """The builder's arrays: of one value, or of several (scheduled on the
+    device, with an infinite tolerance among them)."""
+    from bacon_amd import ivp
+    w = _lv(n)
+    rng = np.random.default_rng(n)
+    w["t_end"], w["tol"], w["t0"] = np.full(n, 0.75), np.full(n, 1e-6), 0.125
+    if fields in ("tol", "all"):
+        w["tol"] = 10.0 ** rng.uniform(-8, -4, n)
+        w["tol"][n // 2] = np.inf
+    if fields in ("t_end", "all"):
+        w["t_end"] = rng.uniform(0.5, 1.5, n)
+    _same(w, ivp.solve_ensemble(L.RK45, dict(w, t0=np.full(n, 0.125))))
