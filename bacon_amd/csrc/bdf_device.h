@@ -53,12 +53,6 @@ __device__ __forceinline__ double dpp_f64(double v) {
         (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, false);
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
-// value of lane l ^ 32, one 32-bit swap
-__device__ __forceinline__ float xor32_f32(float v) {
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    const auto p = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    return __builtin_bit_cast(float, __lane_id() < 32 ? p[1] : p[0]);
-}
 // lane l's value, broadcast (l wave-uniform)
 __device__ __forceinline__ double readlane_lu(double v, int l) {
     const uint64_t b = __builtin_bit_cast(uint64_t, v);
@@ -69,8 +63,20 @@ __device__ __forceinline__ double readlane_lu(double v, int l) {
 __device__ __forceinline__ float readlane_lu(float v, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
-__device__ __forceinline__ double xor32_lu(double v) { return xor32_f64(v); }
-__device__ __forceinline__ float xor32_lu(float v) { return xor32_f32(v); }
+// half hk's value in both halves (hk a constant: one of a swap's results)
+__device__ __forceinline__ double half_lu(double v, int hk) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)b, hi = (uint32_t)(b >> 32);
+    const auto pl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto ph = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __builtin_bit_cast(double, ((uint64_t)ph[hk] << 32) | pl[hk]);
+}
+__device__ __forceinline__ float half_lu(float v, int hk) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v);
+    const auto p = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    const uint32_t w = p[hk];  // (a bit cast of the element itself takes element 0)
+    return __builtin_bit_cast(float, w);
+}
 
 // 1 / a for a pivot of the whole-wave elimination: the hardware reciprocal
 // refined by Newton steps (two for double, one for float), within an ulp or
@@ -86,6 +92,41 @@ __device__ __forceinline__ double pivot_recip(double a) {
 __device__ __forceinline__ float pivot_recip(float a) {
     const float r = __builtin_amdgcn_rcpf(a);
     return fmaf(r, fmaf(-a, r, 1.0f), r);
+}
+
+// d + row_newbcast(r, C) * f by one fma: lane C of each 16-lane row of r is an
+// operand modifier of the multiply-add (through the intrinsic it would be a
+// move before it).  WAIT: the first use of r, and a sum that may go into a lane
+// operation next; the compiler does not insert the wait states of lane
+// operations around inline assembly.
+template <int C, bool WAIT>
+__device__ __forceinline__ double fma_newbcast(double r, double f, double d) {
+    if constexpr (WAIT)
+        asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
+            : "+v"(d) : "v"(r), "v"(f), "n"(C));
+    else
+        asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+            : "+v"(d) : "v"(r), "v"(f), "n"(C));
+    return d;
+}
+template <int C, bool WAIT>
+__device__ __forceinline__ float fma_newbcast(float r, float f, float d) {
+    if constexpr (WAIT)
+        asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
+            : "+v"(d) : "v"(r), "v"(f), "n"(C));
+    else
+        asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+            : "+v"(d) : "v"(r), "v"(f), "n"(C));
+    return d;
+}
+// f(0), ..., f(N - 1) with constant arguments
+template <class F, int... I>
+__device__ __forceinline__ void for_ints(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_ints(F &&f) {
+    for_ints(f, std::make_integer_sequence<int, N>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -632,6 +673,17 @@ struct BdfLane {
     // at the end.  A row that has been a pivot row holds pivot times its
     // normalised values, so later updates stay consistent; this saves the
     // per-step scaling of the pivot row.
+    //
+    // The step was bound by the LDS unit: 64 lanes reading the half row as 8
+    // broadcast b128 loads (8 cycles each) beside its 8 stores, for 16
+    // multiply-adds.  Lane j of a 16-lane row now reads column j alone, one
+    // b64 load, and the multiply-adds take it as their broadcast operand at
+    // the full rate (FP32: at half rate, still the shorter way).  What is left
+    // is the stores (57 % of the LDS unit's cycles) and the vector issue
+    // (60 %).  32,768 Brusselator instances to t = 10: FP64 98.5 -> 83.0 ms,
+    // FP32 60.9 -> 56.2.  With the matrix spread over the wave by columns, one
+    // store of the pivot row in place of 8, the row's choice at run time cost
+    // more than the stores (101 ms).
     __device__ __forceinline__ bool invert_split() {
         LuT b[WJ];
 #pragma unroll
@@ -644,9 +696,8 @@ struct BdfLane {
         int my_col = 0;
         LuT my_inv = (LuT)1;
         LuT *const prow = pivot_row();
-#pragma unroll
-        for (int k = 0; k < W; ++k) {
-            const int hk = k / WJ, kk = k % WJ;
+        for_ints<W>([&](auto column) {
+            constexpr int k = decltype(column)::value, hk = k / WJ, kk = k % WJ;
             const LuT mk = b[kk];
             // half hk holds column k in its own lanes: its reduction is the
             // key (the other half reduces another column, unused), and the
@@ -656,21 +707,28 @@ struct BdfLane {
             const uint32_t key = __builtin_elementwise_max(
                 (uint32_t)__builtin_amdgcn_readlane((int)rm, hk * W),
                 (uint32_t)__builtin_amdgcn_readlane((int)rm, hk * W + 16));
-            const LuT other = xor32_lu(mk);
-            const LuT agk = (h == hk) ? mk : other;
+            const LuT agk = half_lu(mk, hk);
             key_min = __builtin_elementwise_min(key_min, key);
             const int pl = pivot_lane32(key);
             const bool piv = (pl == grp.g);
             if (piv) {
-                used = true;
-                my_col = k;
 #pragma unroll
                 for (int j = 0; j < WJ; ++j) prow[h * WJ + j] = b[j];
-                my_inv = pivot_recip(agk);
             }
+            used = used || piv;
+            my_col = piv ? k : my_col;
             __builtin_amdgcn_wave_barrier();
-            // 1 / pivot straight from the pivot lane (half 0), not via LDS
-            const LuT inv = readlane_lu(my_inv, pl);
+            // lane j of a 16-lane row reads column j of its half
+            const LuT pr = prow[h * WJ + (grp.g & 15)];
+            __builtin_amdgcn_wave_barrier();
+            // 1 / pivot in every lane (the pivot is wave-uniform), while the
+            // row is on its way through LDS
+            const LuT inv = pivot_recip(readlane_lu(mk, hk * W + pl));
+            my_inv = piv ? inv : my_inv;
+            // here, not deferred to the end of the elimination with all the
+            // columns' pivots kept until then
+            asm("" : "+v"(my_inv));
+            asm("" : "+s"(key_min));
             // Every lane updates, so the next column's pivot search can
             // overlap this step's FMAs.  The pivot row's lanes read back
             // their own row and take factor +0: fma(+0, b, b) = b for every
@@ -679,13 +737,19 @@ struct BdfLane {
             // either way).
             const LuT f = agk * inv;
             const LuT nf = piv ? (LuT)0 : -f;
-#pragma unroll
-            for (int j = 0; j < WJ; ++j) b[j] = fma(nf, prow[h * WJ + j], b[j]);
+            // the next column first: its pivot search starts while the others
+            // are updated
+            constexpr int next = (kk + 1) % WJ;
+            b[next] = fma_newbcast<next, true>(pr, nf, b[next]);
+            for_ints<WJ>([&](auto col) {
+                constexpr int j = decltype(col)::value;
+                if constexpr (j != next) b[j] = fma_newbcast<j, false>(pr, nf, b[j]);
+            });
             // column k of the inverse: pivot * (1 / pivot) on the pivot row,
             // -a(g, k) / pivot elsewhere
             if (h == hk) b[kk] = piv ? (LuT)1 : -f;
             __builtin_amdgcn_wave_barrier();
-        }
+        });
         const bool ok = pivot_nonzero32(key_min);
 #pragma unroll
         for (int j = 0; j < WJ; ++j) b[j] *= my_inv;
@@ -1628,9 +1692,11 @@ struct BTag {
     using type = T;
 };
 
-// few: the ensemble has at most three waves per SIMD, so the kernel that is
-// limited to three (and spills less) fits it: 100 (1000, 2000) Brusselator
-// instances to t = 1 1.04 -> 0.95 (1.50 -> 1.46, 2.00 -> 1.94) ms.
+// few: at most five waves per SIMD in all.  The kernel that is limited to three
+// resident ones spills less; a second round of a third of them costs less than
+// the spills up to there: to t = 10 4096 (5000, 6144, 9000) Brusselator
+// instances take 15.8 (18.8, 21.8, 28.3) ms with it against 18.2 (19.2, 22.0,
+// 28.0) with four resident; 256 to t = 4 2.8 against 3.1.
 template <class R, int O, class S, class F>
 static constexpr auto bdf_kernel(bool few) {
     if constexpr (R::W == 32)
@@ -1651,7 +1717,7 @@ static int bdf_launch_shape(const bg_ensemble_desc &d, uint64_t &grid, size_t &b
     int dev = 0;
     BG_HIP_CHECK(hipGetDevice(&dev));
     int per_cu = 0;
-    few = d.n <= (uint64_t)(12 * device_cu_count(dev));
+    few = d.n <= (uint64_t)(20 * device_cu_count(dev));
     BG_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, bdf_kernel<R, O, S, F>(few), 64, 0));
     if (occupancy) *occupancy = per_cu;

@@ -84,3 +84,25 @@ def test_same_bits_in_any_company(gpu, rhs, n):
         for k in ("t", "n_accepted", "n_rejected", "n_newton", "n_lu"):
             assert np.array_equal(p[k], g[k][sel]), k
         assert np.array_equal(p["y"], g["y"][:, sel])
+
+
+@pytest.mark.parametrize("n", [1, 768, 3073, 5120, 5121])
+def test_inverses_of_the_whole_wave_solver(gpu, n):
+    """The 32-component solver around the sizes at which its kernel changes:
+    the same bits as in another ensemble, and the FP32 inverse (an error of
+    about 1e-7 of the correction) leads to the accepted steps and, within 2 %,
+    to the iterations of the FP64 one."""
+    w = W.brusselator(n, cells=16)
+    w["t_end"] = np.full(n, 0.4)
+    g = ivp.solve_ensemble(L.BDF6, w)
+    assert (g["status"] == 0).all()
+    pick = np.unique(np.linspace(0, n - 1, 7).astype(int))
+    p = ivp.solve_ensemble(L.BDF6, _part(w, pick))
+    for k in ("t", "status", "n_accepted", "n_rejected", "n_newton", "n_lu"):
+        assert np.array_equal(p[k], g[k][pick]), k
+    assert np.array_equal(p["y"], g["y"][:, pick])
+    f = ivp.solve_ensemble(L.BDF6, w, lu_bits=32)
+    assert (f["status"] == 0).all()
+    assert np.mean(f["n_accepted"] != g["n_accepted"]) <= 0.01
+    assert abs(f["n_newton"].sum() - g["n_newton"].sum()) <= 0.02 * g["n_newton"].sum()
+    assert np.abs(f["y"] - g["y"]).max() < 1e-5
