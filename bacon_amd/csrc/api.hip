@@ -763,13 +763,11 @@ extern "C" int bg_rk_solve_device(int method, int rhs, int semantics, const bg_e
 
 // ---------------------------------------------------------------------------
 // Allocation-free RK launch.  The persistent launch's workspace (the work
-// counter at [0, 256), the descriptor copy after it) lives in this file-scope
-// device array instead of coming from the stream-ordered allocator.  Each
+// counter) lives in this file-scope device array instead of coming from the stream-ordered allocator.  Each
 // GPU holds its own copy until the process ends; its address is looked up
 // once per device (hipGetSymbolAddress, with that device current) and only
-// that address is handed to kernels.  The setup kernel rewrites the counter
-// and the descriptor at the start of every launch, so nothing carries over
-// from the previous call; calls that overlap on one GPU share the array and
+// that address is handed to kernels.  A launch that uses the counter sets it
+// first, so nothing carries over from the previous call; calls that overlap on one GPU share the array and
 // race.
 // ---------------------------------------------------------------------------
 constexpr size_t kNoAllocScratchBytes = 1024;

@@ -11,7 +11,7 @@
 // Lorenz-63).  Lane g of a group
 // owns component g of every vector (state, guess, residuals, the history of
 // the last O accepted values) and row g of the Jacobian inverse, all in VGPRs.
-// Group collectives use cross-lane shuffles (ds_bpermute); the column sums of
+// Group collectives are DPP moves and lane swaps; the column sums of
 // the Broyden update u = s^T J^-1 go through an LDS transpose (row stride
 // W+1 doubles: conflict-free column reads).  The inverse is Gauss-Jordan with
 // partial pivoting on the rows (implicit, no row swaps); its arithmetic type
@@ -1340,11 +1340,10 @@ struct BdfLane {
 // persistent ensemble kernels
 // ---------------------------------------------------------------------------
 // One instance per wave (the 32-component system).
-// Four waves per SIMD (the LDS limit): the solver is latency-bound (an LDS
-// round trip on every elimination step), and waves hide each other's
-// waits.  On the 32-component Brusselator, 4 waves with 101 VGPRs spilled
-// measured 392 ms against 395 ms for 3 waves with 43 spilled (FP32 inverse:
-// 240 against 248 ms); 3 had beaten 2 by 20 % before.
+// Four waves per SIMD (the LDS limit) hide each other's waits in the
+// elimination, a chain of pivot search, LDS round trip and reciprocal per
+// step.  32,768 Brusselator instances: 82.9 ms with 4 waves and their spills,
+// 85.9 with 3 (up to 20 instances per CU the 3 win: bdf_kernel).
 template <class RHS, int O, class Sem, class LuT, int WAVES>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
     bdf_wave_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter) {

@@ -9,10 +9,11 @@
 
 namespace bg {
 
-// Device workspace of one persistent launch: the work counter at [0, 256),
-// the descriptor copy after it.  A launcher given ws == nullptr takes it from
-// the stream-ordered allocator and frees it on the stream; a caller-owned
-// workspace (graph capture) must hold kLaunchWorkspaceBytes.
+// Device workspace of one persistent launch: the work counter in its first
+// word.  It is used only if the ensemble has more instances than the launch has
+// places for at once.  A launcher given ws == nullptr takes it from the
+// stream-ordered allocator and frees it on the stream; a caller-owned workspace
+// (graph capture) must hold kLaunchWorkspaceBytes.
 constexpr size_t kLaunchWorkspaceBytes = 256 + ((sizeof(bg_ensemble_desc) + 255) & ~(size_t)255);
 
 // Launches of the RK family.  Each returns a BG_* status.

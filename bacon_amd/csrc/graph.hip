@@ -3,9 +3,10 @@
 // For callers that solve the same ensemble layout again and again (parameter
 // sweeps, optimisation loops) the host work of a launch — argument checks,
 // occupancy query, workspace allocation — happens once, at capture.  The
-// graph holds the launch sequence a device entry point issues: the setup
-// kernel (queue counter reset and descriptor copy; a kernel node, so the
-// graph records no memset) and the persistent solve kernel.  For BDF the
+// graph holds the launch sequence a device entry point issues: the persistent
+// solve kernel and, if the ensemble has more instances than it has places for
+// at once, the kernel that sets the queue counter before it (a kernel node, so
+// the graph records no memset).  For BDF the
 // Newton (Broyden) iterations run inside that kernel, so one replay is the
 // whole solve, iterations included.  The workspace is allocated at capture
 // and owned by the graph; replays read the descriptor's device buffers as

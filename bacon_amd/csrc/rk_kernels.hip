@@ -107,7 +107,7 @@ __device__ __forceinline__ int rk_advance(RkLane<RHS, Tab, H> &L, uint32_t &atte
 // wave-uniform exit test (a lane at its end or below dt_min, or the attempt
 // budget that the wave's lanes share until the first could reach its cap);
 // statuses and attempt counts are settled outside it.  Lorenz-63 RK45: 193 ->
-// 171 vector instructions per attempt.
+// 170 vector instructions per attempt.
 template <class RHS, class Tab>
 __global__ void __launch_bounds__(256)
     rk_ensemble_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter,

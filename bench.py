@@ -145,9 +145,9 @@ def graph_replay(cx):
     """One captured graph replay against the eager entry point, on short
     solves where the launch is a visible share of the time: 256 Brusselator
     instances under BDF6 to t = 0.05 (one wave each), and 4096 Lorenz-63
-    instances under RK45 to t = 0.1.  The eager call takes its workspace from
-    the stream-ordered allocator and launches a setup kernel and the solve
-    kernel; the graph owns its workspace and replays both kernels.  Each
+    instances under RK45 to t = 0.1.  Both have
+    a place for every instance at once, so the eager call launches the solve
+    kernel alone, without a workspace, and the graph replays that kernel.  Each
     side: 50 back-to-back launches on one stream, after 3 warm-up launches;
     the replay's outputs are checked bit for bit against the eager solve."""
     from bacon_amd import workloads as W

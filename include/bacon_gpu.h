@@ -225,8 +225,8 @@ int bg_rk_solve_device(int method, int rhs, int semantics, const bg_ensemble_des
 /* The same launch without any allocation: no counterpart in the reference;
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The
- * launch's workspace (work counter and descriptor copy, 1 KiB at most: it
- * does not grow with d->n) is a static device array of the library, one per
+ * launch's workspace (the work counter, 1 KiB at most: it does not grow with
+ * d->n) is a static device array of the library, one per
  * GPU, reused by every call on that GPU: calls that overlap on one GPU race.
  * Same arguments, results and errors as bg_rk_solve_device.  Asynchronous. */
 int bg_rk_solve_device_noalloc(int method, int rhs, int semantics, const bg_ensemble_desc *d,
@@ -242,11 +242,10 @@ int bg_rk_solve_plain_device(int method, int rhs, int semantics, const bg_ensemb
  * stop and an accepted clamped step lands exactly on it. */
 #define BG_PATH_STOPS_ONLY 1u   /* record only landings on stops and the end */
 /* Instance-major buffers: path_t[n][capacity], path_y[n][capacity][dim].
- * Each instance's records are contiguous, so the stores of consecutive
- * steps fill the same cache lines; the default [capacity][n] layout
- * coalesces only while the lanes of a wave record in step, and instances
- * desynchronise within a few steps (measured on 262,144 Lorenz-63
- * instances with every step recorded: 41 ms default, see the bench). */
+ * Each instance's records are contiguous.  The solve writes packed records and
+ * a second kernel lays them out where the records exceed the caches, so the
+ * two layouts take about the same time (262,144 Lorenz-63 instances, every
+ * step into a ring of 64: 8.3 ms default, 9.2 instance-major). */
 #define BG_PATH_INSTANCE_MAJOR 2u
 typedef struct {
     uint32_t capacity;     /* entries per instance (0: count only)             */
@@ -310,9 +309,9 @@ int bg_rk_solve_tuned_device(int method, int rhs, int semantics, const bg_ensemb
 /* ------------------------------------------------------------------------ */
 /* HIP graph capture (no counterpart in the reference)                      */
 /* ------------------------------------------------------------------------ */
-/* One batched solve captured once and replayed: the setup kernel (counter
- * reset, descriptor copy) and the persistent solve kernel, whose BDF Newton
- * iterations run inside it.  The launch workspace is allocated at capture and
+/* One batched solve captured once and replayed: the persistent solve kernel,
+ * whose BDF Newton iterations run inside it, and before it, for ensembles with
+ * more instances than are resident, the kernel that sets the work counter.  The launch workspace is allocated at capture and
  * owned by the graph.  A replay reads the descriptor's device buffers as they
  * hold at replay time.  Replays of one graph must not overlap each other. */
 typedef struct bg_graph bg_graph;
