@@ -617,7 +617,17 @@ struct BdfLane {
         ((xs[K] = grp.template bcast_at<K>(x)), ...);
     }
 
-    // y_g = -(Jinv x)_g with x broadcast through LDS (quads: DPP moves)
+    // SPLIT = 2: component h W/2 + j of v in lane j of each 16-lane row, where
+    // multiply-adds take it as their broadcast operand.  32,768 Brusselator
+    // instances against 16 values per lane through LDS in each product and
+    // update: 82.9 -> 79.4 ms (FP32 inverse 56.2 -> 53.6).
+    __device__ __forceinline__ double half_columns(double v) const {
+        const double o = xor16_f64(v);
+        return (grp.g >> 4) == h ? v : o;
+    }
+
+    // y_g = -(Jinv x)_g with x broadcast through LDS (quads: DPP moves; the
+    // whole wave: half_columns)
     __device__ __forceinline__ double neg_jinv_times(double x) {
         if constexpr (W <= 4) {
             double xs[W];
@@ -627,13 +637,21 @@ struct BdfLane {
             for (int j = 0; j < W; ++j) acc = fma(jinv[j], xs[j], acc);
             return -acc;
         }
-        lds[grp.g] = x;
-        __builtin_amdgcn_wave_barrier();
         double acc = 0.0;
+        if constexpr (SPLIT == 2) {
+            const double xs = half_columns(x);
+            for_ints<WJ>([&](auto col) {
+                constexpr int j = decltype(col)::value;
+                acc = fma_newbcast<j, j == 0 || j == WJ - 1>(xs, jinv[j], acc);
+            });
+            acc += xor32_f64(acc);
+        } else {
+            lds[grp.g] = x;
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int j = 0; j < WJ; ++j) acc = fma(jinv[j], lds[h * WJ + j], acc);
-        if constexpr (SPLIT == 2) acc += xor32_f64(acc);
-        __builtin_amdgcn_wave_barrier();
+            for (int j = 0; j < WJ; ++j) acc = fma(jinv[j], lds[j], acc);
+            __builtin_amdgcn_wave_barrier();
+        }
         return -acc;
     }
 
@@ -1195,11 +1213,17 @@ struct BdfLane {
                 spread(u, us, std::make_integer_sequence<int, W>{});
 #pragma unroll
                 for (int j = 0; j < W; ++j) jinv[j] = fma(us[j], w, jinv[j]);
+            } else if constexpr (SPLIT == 2) {
+                const double us = half_columns(u);
+                for_ints<WJ>([&](auto col) {
+                    constexpr int j = decltype(col)::value;
+                    jinv[j] = fma_newbcast<j, j == 0>(us, w, jinv[j]);
+                });
             } else {
                 lds[grp.g] = u;
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int j = 0; j < WJ; ++j) jinv[j] = fma(lds[h * WJ + j], w, jinv[j]);
+                for (int j = 0; j < WJ; ++j) jinv[j] = fma(lds[j], w, jinv[j]);
                 __builtin_amdgcn_wave_barrier();
             }
             // s = -Jinv_new F (bdf.rs:464-465) without a second product
@@ -1342,8 +1366,9 @@ struct BdfLane {
 // One instance per wave (the 32-component system).
 // Four waves per SIMD (the LDS limit) hide each other's waits in the
 // elimination, a chain of pivot search, LDS round trip and reciprocal per
-// step.  32,768 Brusselator instances: 82.9 ms with 4 waves and their spills,
-// 85.9 with 3 (up to 20 instances per CU the 3 win: bdf_kernel).
+// step.  32,768 Brusselator instances, while the Broyden products still went
+// through LDS: 82.9 ms with 4 waves and their spills, 85.9 with 3 (up to 20
+// instances per CU the 3 win: bdf_kernel).
 template <class RHS, int O, class Sem, class LuT, int WAVES>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
     bdf_wave_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter) {
