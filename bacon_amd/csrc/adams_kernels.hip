@@ -538,9 +538,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                     const double hi = L.tol() / c, lo = 0.1 * hi;
                     ss_hi = hi * hi * (1.0 - 1e-10);
                     ss_lo = lo * lo * (1.0 + 1e-10);
-                    // out of the range in which the margins hold: every step
-                    // by the exact test
-                    if (!(ss_lo > 1e-280 && ss_hi < 1e280)) ss_lo = __builtin_inf();
+                    // out of the range in which the margins hold, or a sign
+                    // that the squares would lose: every step by the exact
+                    // test
+                    if (!(ss_lo > 1e-280 && ss_hi < 1e280 && c > 0.0 && hi > 0.0))
+                        ss_lo = __builtin_inf();
                 }
                 if (4 * __popcll(ballot(slow)) <= waiting) break;
             }

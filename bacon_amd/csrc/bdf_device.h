@@ -222,15 +222,16 @@ struct Grp {
 };
 
 // sqrt(ss) <= bound (OR_EQUAL) or sqrt(ss) < bound, as the rounded square root
-// would decide.  SQUARES: away from the bound the squares decide (a margin of
-// 1e-10 each way, far above their rounding), within it the root itself.  Not
+// would decide.  SQUARES: away from a positive bound the squares decide (a
+// margin of 1e-10 each way, far above their rounding), within it, and for any
+// other bound (the square would lose its sign), the root itself.  Not
 // in the whole-wave solver, whose registers are full: there the branch cost
 // more in spills than the root (27.5 against 26.7 ms, 32,768 instances to t = 2).
 template <bool SQUARES, bool OR_EQUAL>
 __device__ __forceinline__ bool norm_below(double ss, double bound) {
     if constexpr (SQUARES) {
         const double b2 = bound * bound;
-        if (b2 > 1e-290) {
+        if (bound > 1e-145) {
             if (ss < b2 * (1.0 - 1e-10)) return true;
             if (ss > b2 * (1.0 + 1e-10)) return false;
         }
