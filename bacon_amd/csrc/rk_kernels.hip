@@ -15,6 +15,10 @@
 //    stalling the other lanes; an ensemble that fits the resident lanes needs
 //    no counter;
 //  * an optional schedule permutation hands out instances longest-first.
+#include <string.h>
+
+#include <mutex>
+
 #include "bg_device.h"
 #include "bg_internal.h"
 
@@ -404,9 +408,10 @@ __global__ void __launch_bounds__(256)
 }
 
 // The packed records to the caller's arrays: only entries that were written
-// (the first min(records, capacity) of an instance).  A block moves
-// kUnpackSlots entries of 64 instances through LDS, so that it reads runs of
-// kUnpackSlots records and, in the default layout, writes 64 neighbours.
+// (the first min(records, capacity) of an instance) are read and moved.  A
+// block moves kUnpackSlots entries of 64 instances at a time through LDS, so
+// that it reads runs of kUnpackSlots records and, in the default layout, writes
+// 64 neighbours, and stops at the most that any of the 64 has.
 // Bound by HBM: 537 MB in, 537 MB out in 0.21 ms (5.1 TB/s).
 constexpr int kUnpackSlots = 8;
 template <int D>
@@ -415,41 +420,46 @@ __global__ void __launch_bounds__(256)
                        uint64_t n, const bg_path_desc pd) {
     constexpr int W = kRecord<D>, RUN = kUnpackSlots * W;
     __shared__ double tile[64][RUN + 1];
+    __shared__ uint32_t have_of[64];
     const uint32_t capacity = pd.capacity;
     const uint64_t i0 = (uint64_t)blockIdx.x * 64;
-    const uint32_t e0 = blockIdx.y * kUnpackSlots;
-    const uint32_t slots = capacity - e0 < (uint32_t)kUnpackSlots ? capacity - e0 : kUnpackSlots;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t k = threadIdx.x; k < 64 * RUN; k += 256) {
-        const uint32_t i = k / RUN, f = k % RUN;
-        if (i0 + i < n && f < slots * W)
-            tile[i][f] = records[((i0 + i) * capacity + e0) * W + f];
-    }
+    uint32_t have = i0 + lane < n ? n_records[i0 + lane] : 0u;
+    have = have < capacity ? have : capacity;
+    if (wave == 0) have_of[lane] = have;
+    const uint32_t most = wave_max_u32(have);
     __syncthreads();
-    if ((pd.flags & BG_PATH_INSTANCE_MAJOR) != 0) {
-        // consecutive threads: consecutive values of one instance
-        for (uint32_t k = threadIdx.x; k < 64u * kUnpackSlots * (1 + D); k += 256) {
-            const uint32_t i = k / (kUnpackSlots * (1 + D)), r = k % (kUnpackSlots * (1 + D));
-            const uint32_t e = r < kUnpackSlots ? r : (r - kUnpackSlots) / D;
-            if (i0 + i >= n || e >= slots || e0 + e >= n_records[i0 + i]) continue;
-            const uint64_t at = (i0 + i) * capacity + e0 + e;
-            if (r < kUnpackSlots) {
-                pd.path_t[at] = tile[i][e * W];
-            } else {
-                const uint32_t c = (r - kUnpackSlots) % D;
-                pd.path_y[at * D + c] = tile[i][e * W + 1 + c];
+    for (uint32_t e0 = blockIdx.y * kUnpackSlots; e0 < most; e0 += gridDim.y * kUnpackSlots) {
+        for (uint32_t k = threadIdx.x; k < 64 * RUN; k += 256) {
+            const uint32_t i = k / RUN, f = k % RUN;
+            if (e0 + f / W < have_of[i]) tile[i][f] = records[((i0 + i) * capacity + e0) * W + f];
+        }
+        __syncthreads();
+        if ((pd.flags & BG_PATH_INSTANCE_MAJOR) != 0) {
+            // consecutive threads: consecutive values of one instance
+            for (uint32_t k = threadIdx.x; k < 64u * kUnpackSlots * (1 + D); k += 256) {
+                const uint32_t i = k / (kUnpackSlots * (1 + D)), r = k % (kUnpackSlots * (1 + D));
+                const uint32_t e = r < kUnpackSlots ? r : (r - kUnpackSlots) / D;
+                if (e0 + e >= have_of[i]) continue;
+                const uint64_t at = (i0 + i) * capacity + e0 + e;
+                if (r < kUnpackSlots) {
+                    pd.path_t[at] = tile[i][e * W];
+                } else {
+                    const uint32_t c = (r - kUnpackSlots) % D;
+                    pd.path_y[at * D + c] = tile[i][e * W + 1 + c];
+                }
+            }
+        } else {
+            for (uint32_t r = wave; r < kUnpackSlots * (1 + D); r += 4) {
+                const uint32_t e = r / (1 + D), c = r % (1 + D);
+                if (e0 + e >= have) break;
+                const uint64_t at = e0 + e;
+                const double v = tile[lane][e * W + c];
+                if (c == 0) pd.path_t[at * n + i0 + lane] = v;
+                else pd.path_y[(at * D + c - 1) * n + i0 + lane] = v;
             }
         }
-    } else if (i0 + lane < n) {
-        const uint32_t have = n_records[i0 + lane];
-        for (uint32_t r = wave; r < slots * (1 + D); r += 4) {
-            const uint32_t e = r / (1 + D), c = r % (1 + D);
-            if (e0 + e >= have) break;
-            const uint64_t at = e0 + e;
-            const double v = tile[lane][e * W + c];
-            if (c == 0) pd.path_t[at * n + i0 + lane] = v;
-            else pd.path_y[(at * D + c - 1) * n + i0 + lane] = v;
-        }
+        __syncthreads();  // before the next entries overwrite the tile
     }
 }
 
@@ -678,7 +688,63 @@ int rk_launch_path(int method, int rhs, int semantics, uint32_t dim, PathState *
 }
 
 // Sizes between which the path kernel packs its records (see there).
-constexpr size_t kPackedMin = (size_t)32 << 20, kPackedMax = (size_t)8 << 30;
+constexpr size_t kPackedMin = (size_t)32 << 20, kPackedMax = (size_t)1 << 30;
+
+// Workspace of the packed records: a pool of its own on each device that keeps
+// up to kPackedMax bytes from one call to the next.  From the default pool,
+// which gives everything back at each synchronisation, a call paid for fresh
+// memory whenever the driver had to clear it first (28 ms per GB once a program
+// has used as much as the card holds: 15 ms for a ring of 537 MB that is
+// recorded in 1 ms).  The memory goes back when kPoolSpared calls in a row have
+// done without it, or when the pool cannot serve a call.  One lock: the pools
+// are shared by all threads and streams, each allocation is ordered on its
+// caller's stream.
+constexpr uint32_t kPoolSpared = 16;
+struct RecordPool {
+    hipMemPool_t pool;
+    uint32_t spared;
+};
+static std::mutex g_record_mutex;
+static RecordPool g_record_pool[64];
+
+static char *take_records(int dev, size_t bytes, hipStream_t stream) {
+    if (dev < 0 || dev >= 64) return nullptr;
+    std::lock_guard<std::mutex> lk(g_record_mutex);
+    RecordPool &rp = g_record_pool[dev];
+    if (!rp.pool) {
+        hipMemPoolProps props;
+        memset(&props, 0, sizeof props);
+        props.allocType = hipMemAllocationTypePinned;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = dev;
+        hipMemPool_t pool = nullptr;
+        uint64_t keep = kPackedMax;
+        if (hipMemPoolCreate(&pool, &props) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess)
+            (void)hipGetLastError();  // then every call allocates
+        rp.pool = pool;
+    }
+    rp.spared = 0;
+    for (int attempt = 0; attempt < 2; ++attempt) {
+        char *p = nullptr;
+        if (hipMallocFromPoolAsync((void **)&p, bytes, rp.pool, stream) == hipSuccess) return p;
+        (void)hipGetLastError();
+        (void)hipMemPoolTrimTo(rp.pool, 0);
+    }
+    return nullptr;
+}
+
+// A call that needs no records' workspace.
+static void spare_records(int dev) {
+    if (dev < 0 || dev >= 64) return;
+    std::lock_guard<std::mutex> lk(g_record_mutex);
+    RecordPool &rp = g_record_pool[dev];
+    if (rp.pool && rp.spared < kPoolSpared && ++rp.spared == kPoolSpared)
+        (void)hipMemPoolTrimTo(rp.pool, 0);
+}
 
 int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensemble_desc &d,
                             const bg_path_desc &p, hipStream_t stream) {
@@ -696,29 +762,32 @@ int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensembl
         // stops are recorded (there the lanes of a wave write the same entry
         // within a short time), the instances' own lines of an instance-major
         // array fit L2 (two per lane: 3.2 ms against 4.1 packed for 100,000
-        // instances and 1024 entries, 17.0 against 9.2 for 262,144 and 64) or
-        // the stream is being captured (the workspace is the size of the
-        // caller's arrays).
+        // instances and 1024 entries, 17.0 against 9.2 for 262,144 and 64),
+        // the workspace, which is sized by the capacity and not by the records,
+        // exceeds what its pool keeps (200,000 Lotka-Volterra instances, 50
+        // steps each, capacity 1000: see kPackedMax) or the stream is being
+        // captured.
         constexpr int W = kRecord<R::D>;
         const size_t record_bytes = (size_t)d.n * p.capacity * W * sizeof(double);
+        const size_t bytes = record_bytes + d.n * sizeof(uint32_t);
         double *records = nullptr;
         uint32_t *n_records = nullptr;
-        bool pack = !(p.flags & BG_PATH_STOPS_ONLY) && record_bytes >= kPackedMin &&
-                    record_bytes <= kPackedMax &&
-                    !((p.flags & BG_PATH_INSTANCE_MAJOR) && d.n <= 131072);
-        if (pack) {
-            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-            pack = hipStreamIsCapturing(stream, &capturing) == hipSuccess &&
-                   capturing == hipStreamCaptureStatusNone;
-            if (!pack) (void)hipGetLastError();
+        const bool pack = !(p.flags & BG_PATH_STOPS_ONLY) && record_bytes >= kPackedMin &&
+                          bytes <= kPackedMax &&
+                          !((p.flags & BG_PATH_INSTANCE_MAJOR) && d.n <= 131072);
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
+            (void)hipGetLastError();
+            capturing = hipStreamCaptureStatusActive;
         }
-        if (pack) {
-            const size_t bytes = record_bytes + d.n * sizeof(uint32_t);
-            if (hipMallocAsync((void **)&records, bytes, stream) != hipSuccess) {
-                (void)hipGetLastError();  // no room: straight to the caller's arrays
-                records = nullptr;
+        if (capturing == hipStreamCaptureStatusNone) {
+            if (pack) {
+                // no room: straight to the caller's arrays
+                char *ws = take_records(dev, bytes, stream);
+                records = (double *)ws;
+                if (ws) n_records = (uint32_t *)(ws + record_bytes);
             } else {
-                n_records = (uint32_t *)((char *)records + record_bytes);
+                spare_records(dev);
             }
         }
         const bool stops_only = (p.flags & BG_PATH_STOPS_ONLY) != 0;
@@ -745,8 +814,12 @@ int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensembl
             }
             kern<<<(uint32_t)grid, 256, 0, stream>>>(d, p, counter, records, n_records);
             if (records) {
-                const dim3 tiles((uint32_t)((d.n + 63) / 64),
-                                 (p.capacity + kUnpackSlots - 1) / kUnpackSlots);
+                // at most 65,536 blocks, each over as many entries as that takes
+                const uint32_t columns = (uint32_t)((d.n + 63) / 64);
+                uint32_t rows = (p.capacity + kUnpackSlots - 1) / kUnpackSlots;
+                const uint32_t most = columns < 32768u ? 65536u / columns : 2u;
+                // (the y dimension of a grid ends at 65,536)
+                const dim3 tiles(columns, rows < most ? rows : most < 65535u ? most : 65535u);
                 path_unpack_kernel<R::D><<<tiles, 256, 0, stream>>>(records, n_records, d.n, p);
             }
             return hipGetLastError();

@@ -245,7 +245,10 @@ int bg_rk_solve_plain_device(int method, int rhs, int semantics, const bg_ensemb
  * Each instance's records are contiguous.  The solve writes packed records and
  * a second kernel lays them out where the records exceed the caches, so the
  * two layouts take about the same time (262,144 Lorenz-63 instances, every
- * step into a ring of 64: 8.3 ms default, 9.2 instance-major). */
+ * step into a ring of 64: 8.7 ms default and instance-major).  The packed
+ * records' workspace (n * capacity records, at most 1 GiB, else the records go
+ * straight to the caller's arrays) stays with the library for the next call and
+ * is given back after 16 path calls in a row that need none. */
 #define BG_PATH_INSTANCE_MAJOR 2u
 typedef struct {
     uint32_t capacity;     /* entries per instance (0: count only)             */
