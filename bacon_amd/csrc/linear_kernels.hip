@@ -144,11 +144,7 @@ __global__ void __launch_bounds__(64 * LWAVES, Tab::as_built ? 1 : 2)
         dt_min = d.dt_min ? d.dt_min[inst] : d.dt_min_s;
         dt_max = d.dt_max ? d.dt_max[inst] : d.dt_max_s;
         dt = (dt_max + dt_min) * 0.5;  // rk.rs:315
-        // the quotients that div_mid covers (RkLane::set_range)
-        r_lo = tol >= 0x1p-200 && tol <= 0x1p200 && dt_min >= 0x1p-200 && dt_max <= 0x1p200 &&
-                       fabs(end) >= 0x1p-100
-                   ? 1e-8
-                   : __builtin_inf();
+        r_lo = quotient_range(t, end, tol, dt_min, dt_max);
         if constexpr (Tab::as_built) {
 #pragma unroll
             for (int i = 0; i < S; ++i)
@@ -278,7 +274,7 @@ __global__ void __launch_bounds__(64 * LWAVES, Tab::as_built ? 1 : 2)
         double f0 = root8_lds(rr, poly);
         const bool outside = !(rr > r_lo && rr < 65536.0);
         if (__builtin_expect(ballot(outside && step) != 0, 0)) {
-            if (outside) f0 = factor_outside(q2, ss, r_lo, rr);
+            if (outside) f0 = factor_outside(q2, ss, f0, rr);
         }
         const double tang = fma(rr - 1.0, 0.125, 1.0);
         const double f = qmin(f0, tang);
