@@ -49,16 +49,23 @@ CPP_TEST_SRC = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_referen
 CPP_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_reference_ivp.bin")
 
 
+QUEUE_TEST_SRC = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_wave_queue.hip")
+QUEUE_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_wave_queue.bin")
+
+
 def build_cpp_tests(verbose: bool = True) -> str:
     """The C++ restatement of the reference's ivp tests, linked against the
-    library (run on a GPU by tests/test_gpu_cpp.py)."""
-    cmd = ["g++", "-std=c++17", "-O2", "-o", CPP_TEST_BIN, CPP_TEST_SRC,
-           f"-L{HERE}", "-lbacon_gpu", f"-Wl,-rpath,{HERE}", "-Wl,-rpath,$ORIGIN/../../bacon_amd"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"g++ failed:\n{r.stdout}\n{r.stderr}")
-    if verbose:
-        print(f"built {CPP_TEST_BIN}")
+    library, and the work queue's own test (run on a GPU by
+    tests/test_gpu_cpp.py and tests/test_gpu_wave_queue.py)."""
+    for cmd in (["g++", "-std=c++17", "-O2", "-o", CPP_TEST_BIN, CPP_TEST_SRC,
+                 f"-L{HERE}", "-lbacon_gpu", f"-Wl,-rpath,{HERE}",
+                 "-Wl,-rpath,$ORIGIN/../../bacon_amd"],
+                [hipcc(), *HIPFLAGS, "-o", QUEUE_TEST_BIN, QUEUE_TEST_SRC]):
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"{cmd[0]} failed:\n{r.stdout}\n{r.stderr}")
+        if verbose:
+            print(f"built {cmd[cmd.index('-o') + 1]}")
     return CPP_TEST_BIN
 
 

@@ -752,7 +752,8 @@ struct WaveQueue {
     }
 
     // the next instance for every lane that wants one, -1 if there is none;
-    // pos: its schedule position
+    // pos: its schedule position (the other lanes' stays what it was: they are
+    // still at work on theirs)
     __device__ __forceinline__ int64_t next(uint32_t *counter, uint32_t n, const int32_t *order,
                                             bool want, uint32_t &pos) {
         const uint32_t lane = __lane_id();
@@ -761,8 +762,8 @@ struct WaveQueue {
         const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
         const uint32_t avail = end - base;
         bool have = want && rank < avail;
-        pos = base + rank;
-        int32_t idx = order ? __shfl(entry, (int)((pos - first) & 63u)) : (int32_t)pos;
+        uint32_t at = base + rank;
+        int32_t idx = order ? __shfl(entry, (int)((at - first) & 63u)) : (int32_t)at;
         if (cnt <= avail) {
             base += cnt;
         } else if (open) {
@@ -785,17 +786,18 @@ struct WaveQueue {
             end = open ? b + size : n;
             first = b;
             if (order) entry = b + lane < end ? gptr(order)[b + lane] : 0;
-            const uint32_t at = rank - avail;
-            const int32_t other = order ? __shfl(entry, (int)(at & 63u)) : (int32_t)(b + at);
+            const uint32_t k = rank - avail;
+            const int32_t other = order ? __shfl(entry, (int)(k & 63u)) : (int32_t)(b + k);
             if (want && rank >= avail) {
-                pos = b + at;
+                at = b + k;
                 idx = other;
-                have = pos < end;
+                have = at < end;
             }
             base = lacking < end - b ? b + lacking : end;
         } else {
             base = end;
         }
+        if (want) pos = at;
         return have ? (int64_t)idx : -1;
     }
 };
