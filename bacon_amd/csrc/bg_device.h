@@ -738,9 +738,11 @@ struct WaveQueue {
     bool open;            // the counter may hold more
     uint32_t run;         // length of the next run
     uint32_t ticks;       // loop iterations since the last claim
+    uint32_t waves;       // waves that share the queue
 
-    __device__ __forceinline__ WaveQueue(const uint32_t *counter)
-        : base(0), end(0), first(0), entry(0), open(counter != nullptr), run(1), ticks(0) {}
+    __device__ __forceinline__ WaveQueue(const uint32_t *counter, uint32_t blocks = gridDim.x)
+        : base(0), end(0), first(0), entry(0), open(counter != nullptr), run(1), ticks(0),
+          waves(blocks * (blockDim.x >> 6)) {}
 
     __device__ __forceinline__ bool drained() const { return !open && base >= end; }
 
@@ -768,7 +770,6 @@ struct WaveQueue {
             base += cnt;
         } else if (open) {
             const uint32_t lacking = cnt - avail;
-            const uint32_t waves = gridDim.x * (blockDim.x >> 6);
             const uint32_t left = n - (end ? end : waves << 6);
             const uint32_t share = left >> (33 - __builtin_clz(waves));
             if (ticks < 128u)

@@ -16,6 +16,39 @@ namespace bg {
 // (graph capture) must hold kLaunchWorkspaceBytes.
 constexpr size_t kLaunchWorkspaceBytes = 256 + ((sizeof(bg_ensemble_desc) + 255) & ~(size_t)255);
 
+// Resident waves per CU of the RK ensemble kernel where the caller leaves them
+// to the library.  In waves, so that the block size does not change them.
+//
+// Waves on a SIMD are served oldest first, so with more than two the youngest
+// crawl (third wave: 2 us an attempt against the first one's 0.4) and end late
+// with what they started early; fewer than two leave issue slots idle.
+// Two per SIMD, then, where instances differ and there are many of them (2^20
+// Lorenz-63 of end times and tolerances of their own, longest first: 57.5 / 49.5
+// / 54.1 / 60.1 / 63.6 ms at 1 .. 5; 2^20 of equal ones 21.1 / 18.7 / 20.2 / 18.9
+// / 19.2), three for scalar bounds, which also hides the refills of short
+// instances (10^6 Lotka-Volterra: 1.21 / 0.97 / 0.82 / 1.12 / 1.09 ms).
+// An ensemble that two waves per SIMD would run in up to two rounds is better
+// off with three if its instances are alike, and with two if not: the counter
+// kernel looks (`look`; 262,144 Lorenz-63, two / three: alike 7.2 / 5.8 ms, end
+// times from 5 to 10 6.0 / 5.5 or longest first 4.7 / 4.3, from 1 to 10 5.0 / 5.0
+// and 3.2 / 3.4, tolerances over a decade 10.7 / 10.0 and 8.5 / 8.0, over three
+// 26.9 / 28.7 and 15.5 / 17.2).  alike: predicted costs within a factor of three.
+constexpr uint32_t kRkWavesFew = 8, kRkWavesMany = 12;
+inline uint32_t rk_default_waves(bool arrays, uint64_t n, int n_cu, bool &look) {
+    const uint64_t few = (uint64_t)kRkWavesFew * 64 * (uint64_t)n_cu;
+    look = arrays && n > few && n <= 2 * few;
+    return arrays && !look ? kRkWavesFew : kRkWavesMany;
+}
+// Blocks per CU that hold so many waves (the nearest number, at least one).
+// Three waves per SIMD do not come out of blocks of two waves, which spread
+// unevenly (262,144 Lorenz-63 in 3 .. 8 blocks: 7.0 / 7.0 / 6.9 / 6.9 / 6.5 /
+// 5.5 ms; blocks of one, three and four waves: 5.8): four.
+inline uint32_t blocks_of_waves(uint32_t waves, uint32_t block) {
+    if (block == 128 && waves == kRkWavesMany) waves = 16;
+    const uint32_t b = (waves * 64 + block / 2) / block;
+    return b ? b : 1u;
+}
+
 // Launches of the RK family.  Each returns a BG_* status.
 int rk_launch_ensemble(int method, int rhs, int semantics, const bg_ensemble_desc &d,
                        const bg_launch &launch, hipStream_t stream, void *ws = nullptr);

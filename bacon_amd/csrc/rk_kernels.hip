@@ -116,12 +116,15 @@ template <class RHS, class Tab>
 __global__ void __launch_bounds__(256)
     rk_ensemble_kernel(const bg_ensemble_desc, uint32_t *__restrict__ counter,
                        uint32_t refill_min, uint32_t prio_cutoff) {
+    // the counter kernel may have set fewer blocks to work than were launched
+    const uint32_t blocks = counter ? counter[1] : gridDim.x;
+    if (blockIdx.x >= blocks) return;
     r8_init();
     const karg_desc dv = kernarg_desc();
     RkLane<RHS, Tab, true> L;
     const uint32_t cap = attempt_cap(dv->max_attempts);
     uint32_t budget = cap;  // attempts until a lane could reach the cap
-    WaveQueue queue(counter);
+    WaveQueue queue(counter, blocks);
     uint32_t pos = blockIdx.x * blockDim.x + threadIdx.x;
     int64_t inst = queue.start(dv->n, dv->order);
     bool take = inst >= 0;
@@ -545,9 +548,46 @@ __global__ void __launch_bounds__(64)
 }
 
 // Work-queue start: the lanes' own positions are taken (a kernel rather than
-// a memset so the launch sequence stays capturable).
-__global__ void rk_counter_kernel(uint32_t *counter, uint32_t lanes) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *counter = lanes;
+// a memset so the launch sequence stays capturable).  counter[1]: the blocks at
+// work.
+__global__ void rk_counter_kernel(uint32_t *counter, uint32_t blocks, uint32_t block) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+        counter[0] = blocks * block;
+        counter[1] = blocks;
+    }
+}
+
+// The same with the choice of rk_default_waves: `many` blocks if the instances
+// are alike, by the predicted cost (t_end - t0) tol^(-1/4) of 1,024 of them (its
+// fourth power: no root), else `few`.
+__global__ void __launch_bounds__(1024)
+    rk_look_kernel(uint32_t *counter, uint32_t few, uint32_t many, uint32_t block,
+                   const bg_ensemble_desc d) {
+    const uint64_t i = (uint64_t)threadIdx.x * d.n / 1024;
+    const double t0 = d.t0 ? d.t0[i] : d.t0_s, end = d.t_end ? d.t_end[i] : d.t_end_s;
+    const double tol = d.tol ? d.tol[i] : d.tol_s;
+    const double span2 = (end - t0) * (end - t0);
+    double lo = span2 * span2 / tol, hi = lo;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, m));
+        hi = fmax(hi, __shfl_xor(hi, m));
+    }
+    __shared__ double lows[16], highs[16];
+    if (__lane_id() == 0) {
+        lows[threadIdx.x >> 6] = lo;
+        highs[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) {
+            lo = fmin(lo, lows[w]);
+            hi = fmax(hi, highs[w]);
+        }
+        const uint32_t blocks = hi <= 81.0 * lo ? many : few;
+        counter[0] = blocks * block;
+        counter[1] = blocks;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -620,37 +660,38 @@ int rk_launch_ensemble(int method, int rhs, int semantics, const bg_ensemble_des
         int per_cu = 0;
         BG_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, rk_ensemble_kernel<R, T>, (int)block, 0));
-        // Default resident blocks.  Waves on a SIMD are served oldest first, so
-        // with more than two the youngest crawl (third wave: 2 us an attempt
-        // against the first one's 0.4) and end late with what they started
-        // early; fewer than two leave issue slots idle.  Two when the
-        // instances' end times or tolerances differ (2^20 Lorenz-63, longest
-        // first: 57 / 52 / 57 / 59 / 61 ms at 1 .. 5 blocks per CU), three when
-        // they do not, which also hides the refills of short instances (10^6
-        // Lotka-Volterra: 3.1 / 2.5 / 2.5 / 2.8 / 2.9 ms; 200,000 plain
-        // Lorenz-63: 5.1 / 4.9 / 4.6 / 5.3 / 5.5 ms).
-        const int want = lc.blocks_per_cu ? (int)lc.blocks_per_cu : (d.tol || d.t_end ? 2 : 3);
-        if (want < per_cu) per_cu = want;
+        const int n_cu = device_cu_count(dev);
+        bool look = false;
+        const uint32_t waves = rk_default_waves(d.t0 || d.t_end || d.tol, d.n, n_cu, look);
+        const uint32_t want = lc.blocks_per_cu ? lc.blocks_per_cu : blocks_of_waves(waves, block);
         if (per_cu < 1) per_cu = 1;
-        uint64_t grid = (uint64_t)per_cu * (uint64_t)device_cu_count(dev);
         const uint64_t need = (d.n + block - 1) / block;
-        if (grid > need) grid = need;
+        auto grid_of = [&](uint32_t blocks) -> uint64_t {
+            const uint64_t g = (blocks < (uint32_t)per_cu ? blocks : (uint64_t)per_cu) * (uint64_t)n_cu;
+            return g < need ? g : need;
+        };
+        const uint64_t grid = grid_of(want);
+        const uint64_t few =
+            look && !lc.blocks_per_cu ? grid_of(blocks_of_waves(kRkWavesFew, block)) : grid;
         const uint32_t refill_min = lc.refill_min ? lc.refill_min : 1u;
         // a lane for every instance: no queue, no workspace
-        const bool queue = d.n > grid * block;
+        const bool queue = d.n > few * block;
         char *ws = (char *)ws_in;
         if (queue) {
             if (!ws_in) BG_HIP_CHECK(hipMallocAsync((void **)&ws, kLaunchWorkspaceBytes, stream));
-            rk_counter_kernel<<<1, 64, 0, stream>>>((uint32_t *)ws, (uint32_t)(grid * block));
+            if (few < grid)
+                rk_look_kernel<<<1, 1024, 0, stream>>>((uint32_t *)ws, (uint32_t)few,
+                                                       (uint32_t)grid, block, d);
+            else
+                rk_counter_kernel<<<1, 64, 0, stream>>>((uint32_t *)ws, (uint32_t)grid, block);
         }
-        // With a schedule the longest instances are the first ones, and the
-        // waves that hold them go first (the older waves do anyway; once they
-        // have finished theirs they give way to the younger ones that still
-        // have theirs to run): 52.5 -> 49.1 ms on the workload above with the
-        // first three quarters of the lanes' positions, 49.7 with all of them,
-        // 51.5 with half.
+        // With a schedule the longest instances are the first ones: the waves
+        // that still hold one of those that they started with go first (the
+        // older waves do anyway; once they have finished theirs they give way to
+        // the younger ones that have not): 2^20 Lorenz-63 of bounds of their own
+        // 54.9 -> 49.5 ms, 50.4 with the first three quarters of the positions.
         const uint32_t prio = lc.prio_cutoff ? lc.prio_cutoff
-                              : d.order && queue ? (uint32_t)(grid * block / 4 * 3) : 0u;
+                              : d.order && queue ? (uint32_t)(few * block) : 0u;
         rk_ensemble_kernel<R, T><<<(uint32_t)grid, block, 0, stream>>>(
             d, queue ? (uint32_t *)ws : nullptr, refill_min, prio);
         const hipError_t launched = hipGetLastError();
@@ -810,7 +851,7 @@ int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensembl
             if (d.n > grid * 256) {
                 e = hipMallocAsync((void **)&counter, kLaunchWorkspaceBytes, stream);
                 if (e != hipSuccess) return e;
-                rk_counter_kernel<<<1, 64, 0, stream>>>(counter, (uint32_t)(grid * 256));
+                rk_counter_kernel<<<1, 64, 0, stream>>>(counter, (uint32_t)grid, 256u);
             }
             kern<<<(uint32_t)grid, 256, 0, stream>>>(d, p, counter, records, n_records);
             if (records) {
