@@ -284,7 +284,15 @@ int rk_autotune(int method, int rhs, int semantics, const bg_ensemble_desc &din,
         BG_TRY(hipMallocAsync((void **)&order, n * sizeof(int32_t), stream));
         if ((rc = schedule(tn, d, order, stream)) != BG_OK) break;
         d.order = order;
-        const uint32_t cand[][2] = {{256, 0}, {256, 4}, {256, 3}, {256, 2}, {128, 6}, {64, 12}};
+        // The default, the occupancy limit (more blocks than fit are as many as
+        // fit) and, of the shapes that the default may stand for, the other one.
+        bool look = false;
+        int dev = 0;
+        BG_TRY(hipGetDevice(&dev));
+        const uint32_t waves =
+            rk_default_waves(d.t0 || d.t_end || d.tol, n, device_cu_count(dev), look);
+        const uint32_t other = waves == kRkWavesFew ? 3u : 2u;
+        const uint32_t cand[][2] = {{256, 0}, {256, 8}, {256, 4}, {256, other}, {128, 4}, {64, 8}};
         double best = 1e300;
         for (const auto &c : cand) {
             bg_launch lc;

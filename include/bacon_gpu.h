@@ -192,11 +192,18 @@ void bg_ensemble_destroy(bg_ensemble *e);
 
 /* Launch shape chosen by the autotuner (zeros = library defaults). */
 typedef struct {
-    uint32_t block;           /* threads per block (multiple of 64)          */
-    uint32_t blocks_per_cu;   /* persistent blocks per CU (0 = occupancy)    */
+    uint32_t block;           /* threads per block (multiple of 64, at most
+                                 256; 0 = 256)                               */
+    uint32_t blocks_per_cu;   /* persistent blocks per CU, at most as many as
+                                 fit (0 = two or three waves per SIMD, by the
+                                 number of instances and whether their bounds
+                                 differ)                                     */
     uint32_t refill_min;      /* refill a wave once this many lanes are idle */
     uint32_t prio_cutoff;     /* waves holding one of the first prio_cutoff
-                                 scheduled instances run at raised priority */
+                                 scheduled instances run at raised priority
+                                 (0 = the positions that the lanes start with,
+                                 if there is an order and more instances than
+                                 lanes; from n on all waves have the same)   */
 } bg_launch;
 
 typedef struct {
