@@ -94,25 +94,41 @@ __device__ __forceinline__ float pivot_recip(float a) {
     return fmaf(r, fmaf(-a, r, 1.0f), r);
 }
 
-// d + row_newbcast(r, C) * f by one fma: lane C of each 16-lane row of r is an
-// operand modifier of the multiply-add (through the intrinsic it would be a
-// move before it).  WAIT: the first use of r, and a sum that may go into a lane
-// operation next; the compiler does not insert the wait states of lane
-// operations around inline assembly.
-template <int C, bool WAIT>
+// The compiler does not insert the wait states of lane operations around inline
+// assembly.  lane_operand: v as the broadcast operand of fma_newbcast, two wait
+// states after the instruction that wrote it; every use of the result comes
+// after them, in whatever order the multiply-adds are scheduled (each with a
+// wait of its own in one of them, ilp-first schedules put others before it).
+// `with`, the other factor, is taken through it too where v comes from memory:
+// the wait for v then does not hold up what computes the factor.
+template <class T>
+__device__ __forceinline__ T lane_operand(T v) {
+    asm("s_nop 1" : "+v"(v));
+    return v;
+}
+template <class T>
+__device__ __forceinline__ T lane_operand(T v, T &with) {
+    asm("s_nop 1" : "+v"(v), "+v"(with));
+    return v;
+}
+// d + row_newbcast(r, C) * f by one fma: lane C of each 16-lane row of r, a
+// lane_operand, is an operand modifier of the multiply-add (through the
+// intrinsic it would be a move before it).  TO_LANES: the sum may go into a lane
+// operation next.
+template <int C, bool TO_LANES>
 __device__ __forceinline__ double fma_newbcast(double r, double f, double d) {
-    if constexpr (WAIT)
-        asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
+    if constexpr (TO_LANES)
+        asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
             : "+v"(d) : "v"(r), "v"(f), "n"(C));
     else
         asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
             : "+v"(d) : "v"(r), "v"(f), "n"(C));
     return d;
 }
-template <int C, bool WAIT>
+template <int C, bool TO_LANES>
 __device__ __forceinline__ float fma_newbcast(float r, float f, float d) {
-    if constexpr (WAIT)
-        asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
+    if constexpr (TO_LANES)
+        asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
             : "+v"(d) : "v"(r), "v"(f), "n"(C));
     else
         asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
@@ -640,10 +656,10 @@ struct BdfLane {
         }
         double acc = 0.0;
         if constexpr (SPLIT == 2) {
-            const double xs = half_columns(x);
+            const double xs = lane_operand(half_columns(x));
             for_ints<WJ>([&](auto col) {
                 constexpr int j = decltype(col)::value;
-                acc = fma_newbcast<j, j == 0 || j == WJ - 1>(xs, jinv[j], acc);
+                acc = fma_newbcast<j, j == WJ - 1>(xs, jinv[j], acc);
             });
             acc += xor32_f64(acc);
         } else {
@@ -738,7 +754,7 @@ struct BdfLane {
             my_col = piv ? k : my_col;
             __builtin_amdgcn_wave_barrier();
             // lane j of a 16-lane row reads column j of its half
-            const LuT pr = prow[h * WJ + (grp.g & 15)];
+            const LuT from_lds = prow[h * WJ + (grp.g & 15)];
             __builtin_amdgcn_wave_barrier();
             // 1 / pivot in every lane (the pivot is wave-uniform), while the
             // row is on its way through LDS
@@ -755,10 +771,11 @@ struct BdfLane {
             // NaN instead of staying infinite: the inverse is not finite
             // either way).
             const LuT f = agk * inv;
-            const LuT nf = piv ? (LuT)0 : -f;
+            LuT nf = piv ? (LuT)0 : -f;
             // the next column first: its pivot search starts while the others
             // are updated
             constexpr int next = (kk + 1) % WJ;
+            const LuT pr = lane_operand(from_lds, nf);
             b[next] = fma_newbcast<next, true>(pr, nf, b[next]);
             for_ints<WJ>([&](auto col) {
                 constexpr int j = decltype(col)::value;
@@ -1215,10 +1232,10 @@ struct BdfLane {
 #pragma unroll
                 for (int j = 0; j < W; ++j) jinv[j] = fma(us[j], w, jinv[j]);
             } else if constexpr (SPLIT == 2) {
-                const double us = half_columns(u);
+                const double us = lane_operand(half_columns(u));
                 for_ints<WJ>([&](auto col) {
                     constexpr int j = decltype(col)::value;
-                    jinv[j] = fma_newbcast<j, j == 0>(us, w, jinv[j]);
+                    jinv[j] = fma_newbcast<j, false>(us, w, jinv[j]);
                 });
             } else {
                 lds[grp.g] = u;
