@@ -411,15 +411,19 @@ __device__ __forceinline__ double div_mid(double a, double b) {
 }
 
 // The controller's factor before the tangent bound for a quotient r = q2 / ss
-// (div_mid's) outside (r_lo, 65536); f0: the root of r.  Either r_lo is +inf,
-// for an instance whose q2 may leave div_mid's range (RkLane::set_range): then
-// this attempt's q2 decides whether r and f0 stand.  Or the clamps
-// delta <= 0.1 / delta >= 4 apply (r <= 1e-8 / r >= 65536, where only the
-// quotient's size matters), or r is NaN.  What is left takes the IEEE division
-// and a root of its own.  1,024 Lorenz-63 instances to t = 10, 1.8 ms, take 2.2
-// with no lower step bound; 2.6 with the division and the second root each time.
-__device__ __forceinline__ double factor_outside(double q2, double ss, double f0, double &r) {
-    if (q2 >= kMidLo && q2 <= kMidHi) {
+// (div_mid's) outside (r_lo, 65536); f0: the root of r.  Either the clamp
+// delta >= 4 applies (only the quotient's size matters): the first test, since
+// an instance whose steps stay at dt_max is here on every attempt.  Or r_lo is
+// +inf, for an instance whose q2 may leave div_mid's range (RkLane::set_range):
+// then this attempt's q2 decides whether r and f0 stand.  Or the clamp
+// delta <= 0.1 applies (r <= 1e-8), or r is NaN.  What is left takes the IEEE
+// division and a root of its own.  1,024 Lorenz-63 instances to t = 10, 1.8 ms,
+// take 2.2 with no lower step bound; 2.6 with the division and the second root
+// each time.
+__device__ __forceinline__ double factor_outside(double q2, double ss, double r_lo, double f0,
+                                                 double &r) {
+    if (r >= 65536.0 && r_lo < 1.0) return 4.0;
+    if (r_lo > 1.0 && q2 >= kMidLo && q2 <= kMidHi) {
         if (r >= 65536.0) return 4.0;
         if (r > 1e-8) return f0;
     }
@@ -632,7 +636,7 @@ struct RkLane {
         }
         const bool outside = !(r > r_lo && r < 65536.0);
         if (__builtin_expect(ballot(outside) != 0, 0)) {
-            if (outside) f0 = factor_outside(q2, ss, f0, r);
+            if (outside) f0 = factor_outside(q2, ss, r_lo, f0, r);
         }
         // near r = 1 the sign of delta - 1 ~ (r - 1)/8 is far below root8's
         // error: bound by the tangent 1 + (r - 1)/8 (r^(1/8) is concave, the

@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(64 * LWAVES, Tab::as_built ? 1 : 2)
         double f0 = root8_lds(rr, poly);
         const bool outside = !(rr > r_lo && rr < 65536.0);
         if (__builtin_expect(ballot(outside && step) != 0, 0)) {
-            if (outside) f0 = factor_outside(q2, ss, f0, rr);
+            if (outside) f0 = factor_outside(q2, ss, r_lo, f0, rr);
         }
         const double tang = fma(rr - 1.0, 0.125, 1.0);
         const double f = qmin(f0, tang);
