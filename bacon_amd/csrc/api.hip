@@ -766,12 +766,12 @@ extern "C" int bg_rk_solve_device(int method, int rhs, int semantics, const bg_e
 
 // ---------------------------------------------------------------------------
 // Allocation-free RK launch.  The persistent launch's workspace (the work
-// counter) lives in this file-scope device array instead of coming from the stream-ordered allocator.  Each
-// GPU holds its own copy until the process ends; its address is looked up
-// once per device (hipGetSymbolAddress, with that device current) and only
-// that address is handed to kernels.  A launch that uses the counter sets it
-// first, so nothing carries over from the previous call; calls that overlap on one GPU share the array and
-// race.
+// counter) lives in this file-scope device array instead of coming from the
+// stream-ordered allocator.  Each GPU holds its own copy until the process
+// ends; its address is looked up once per device (hipGetSymbolAddress, with
+// that device current) and only that address is handed to kernels.  A launch
+// that uses the counter sets it first, so nothing carries over from the previous
+// call; calls that overlap on one GPU share the array and race.
 // ---------------------------------------------------------------------------
 constexpr size_t kNoAllocScratchBytes = 1024;
 static_assert(kLaunchWorkspaceBytes <= kNoAllocScratchBytes,

@@ -10,11 +10,12 @@
 namespace bg {
 
 // Device workspace of one persistent launch: the work counter in its first
-// word.  It is used only if the ensemble has more instances than the launch has
+// word and, for the RK ensemble, the number of blocks at work in its second.
+// It is used only if the ensemble has more instances than the launch has
 // places for at once.  A launcher given ws == nullptr takes it from the
 // stream-ordered allocator and frees it on the stream; a caller-owned workspace
 // (graph capture) must hold kLaunchWorkspaceBytes.
-constexpr size_t kLaunchWorkspaceBytes = 256 + ((sizeof(bg_ensemble_desc) + 255) & ~(size_t)255);
+constexpr size_t kLaunchWorkspaceBytes = 256;
 
 // Resident waves per CU of the RK ensemble kernel where the caller leaves them
 // to the library.  In waves, so that the block size does not change them.

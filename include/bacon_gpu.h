@@ -321,9 +321,10 @@ int bg_rk_solve_tuned_device(int method, int rhs, int semantics, const bg_ensemb
 /* ------------------------------------------------------------------------ */
 /* One batched solve captured once and replayed: the persistent solve kernel,
  * whose BDF Newton iterations run inside it, and before it, for ensembles with
- * more instances than are resident, the kernel that sets the work counter.  The launch workspace is allocated at capture and
- * owned by the graph.  A replay reads the descriptor's device buffers as they
- * hold at replay time.  Replays of one graph must not overlap each other. */
+ * more instances than are resident, the kernel that sets the work counter.  The
+ * launch workspace is allocated at capture and owned by the graph.  A replay
+ * reads the descriptor's device buffers as they hold at replay time.  Replays of
+ * one graph must not overlap each other. */
 typedef struct bg_graph bg_graph;
 int bg_graph_capture_rk(int method, int rhs, int semantics, const bg_ensemble_desc *d,
                         const bg_launch *launch, bg_graph **out);
