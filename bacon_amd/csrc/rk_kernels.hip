@@ -801,10 +801,12 @@ int rk_launch_path_ensemble(int method, int rhs, int semantics, const bg_ensembl
         // Packed records when the caller's arrays are larger than the chip's
         // L2 (below that the lines stay until they are full), unless only
         // stops are recorded (there the lanes of a wave write the same entry
-        // within a short time), the instances' own lines of an instance-major
-        // array fit L2 (two per lane: 3.2 ms against 4.1 packed for 100,000
-        // instances and 1024 entries, 17.0 against 9.2 for 262,144 and 64),
-        // the workspace, which is sized by the capacity and not by the records,
+        // within a short time), the array is instance-major and small (its
+        // instances' lines, two per lane, fit L2 up to some 10^5 of them; at
+        // 131,072 and 128 entries short paths take 0.32 ms direct and 0.41
+        // packed, rings that wrap 20 times 7.3 and 5.1, which the host cannot
+        // tell apart; at 20,000 0.17 and 0.23, 2.3 and 2.2; at 262,144 and 64
+        // entries 17 and 8.7), the workspace, which is sized by the capacity and not by the records,
         // exceeds what its pool keeps (200,000 Lotka-Volterra instances, 50
         // steps each, capacity 1000: see kPackedMax) or the stream is being
         // captured.

@@ -86,7 +86,7 @@ BYTES_PER_INSTANCE = 8 * 8 + 4 + 8 * 4 + 4 + 8
 # HBM bytes per launch measured with rocprofv3 FETCH_SIZE and WRITE_SIZE (each
 # scaled by a 1 GiB copy-kernel calibration); see
 # profiles/rk_ensemble_lorenz_2p20.md
-MEASURED_TRAFFIC_BYTES = 1.065e9 + 0.237e9
+MEASURED_TRAFFIC_BYTES = 1.055e9 + 0.212e9
 
 
 _BASELINE_ORACLE = None
@@ -848,8 +848,8 @@ def main():
                "frac_of_fp64_peak": int(cl.sum()) * FLOPS_ATTEMPT_LINEAR / kern_l / 1e12
                                     / PEAK_FP64_TFLOPS,
                "max_abs_err_vs_closed_form": float(np.abs(yl - ye).max()),
-               "mfma_utilisation_rocprof": 0.78,
-               "hbm_traffic_bytes_rocprof": 68.4e6 + 68.6e6,
+               "mfma_utilisation_rocprof": 0.86,
+               "hbm_traffic_bytes_rocprof": 460e6 + 266e6,
                "rocprof_source": "profiles/linear_mfma_65536.md (rocprofv3 --pmc runs of "
                                  "this workload; constants here, not measured in this run)",
                "algorithmic_hbm_bytes": nl * LIN_N * 8 * 2 + nl * 24}
